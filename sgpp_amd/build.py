@@ -17,7 +17,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 
 HIP_SOURCES = ["meval_kernels.hip", "meval_count.hip", "subspace_kernels.hip", "solver_kernels.hip",
-               "server.hip"]
+               "server.hip", "tree_runtime.hip", "tree_f32_linear.hip", "tree_f32_modlinear.hip",
+               "tree_f64_linear.hip", "tree_f64_modlinear.hip"]
 CPP_SOURCES = ["grid.cpp", "operation_hip.cpp", "learner.cpp", "capi.cpp", "server_capi.cpp"]
 
 INCLUDES = ["-I" + CSRC, "-I" + os.path.join(CSRC, "include"),

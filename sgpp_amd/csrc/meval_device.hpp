@@ -80,6 +80,9 @@ std::vector<int32_t> grid_order(const std::vector<double>& li, const std::vector
 template <typename T>
 std::vector<T> tile_boxes(const std::vector<double>& li, size_t npad, size_t n, size_t d);
 
+struct TreeGrid;     // tree_device.hpp
+struct TreeProgram;
+
 class DeviceMultiEval {
  public:
   // data_rowmajor: M x d, FP64 row-major (the caller's DataMatrix layout).
@@ -178,6 +181,35 @@ class DeviceMultiEval {
   const T* group_boxes() const {
     return static_cast<const T*>(sizeof(T) == sizeof(double) ? WB64_ : WB32_);
   }
+  // refuses a no-allocation call whose weights and one row of partials (of
+  // value_bytes and FP64) exceed the scratch
+  void check_scratch(const MultScratch& ext, size_t value_bytes) const;
+  // the subspace tree (tree_runtime.hip): set_tree uploads a grid's programs
+  // (false: a grid the walks do not cover)
+  struct TreePlan {
+    void* recs = nullptr;    size_t recs_cap = 0;
+    void* chunks = nullptr;  size_t chunks_cap = 0;
+    void* groups = nullptr;  size_t groups_cap = 0;
+    int nchunks = 0, ngroups = 0;
+    int lds = 0;        // bytes of the largest chunk's tables
+    bool wide = false;  // several data points per lane
+  };
+  bool set_tree(const TreeGrid& g, bool multT);
+  // Kernels that evaluate a direction: the algorithm's own or the
+  // subspace tree's
+  enum class Path { Own, Tree };
+  bool set_paths(const TreeGrid* tree, const std::vector<double>& li,
+                 const std::vector<uint32_t>& pmask);
+  bool tree_pays(const TreeGrid& g, const std::vector<double>& li,
+                 const std::vector<uint32_t>& pmask) const;
+  template <typename T>
+  void set_tree_plans(const TreeGrid& g, bool multT);
+  void upload_tree(const TreeProgram& p, TreePlan& plan, int entry_bytes);
+  template <typename T>
+  void run_tree_mult(const double* d_alpha, double* d_result, hipEvent_t* tev,
+                     const MultScratch* ext = nullptr);
+  template <typename T>
+  void run_tree_multT(const double* d_y, double* d_result, hipEvent_t* tev);
   // the subspace algorithm (subspace_kernels.hip)
   void set_grid_subspace(const uint32_t* level, const uint32_t* index, size_t N);
   void run_subspace_mult(const double* d_alpha, double* d_result, hipEvent_t* tev);
@@ -231,6 +263,16 @@ class DeviceMultiEval {
   void* sub_tw_ = nullptr;    size_t sub_tw_cap_ = 0;
   void* sub_chunk_ = nullptr; size_t sub_chunk_cap_ = 0;  // multTranspose chunks
   int nchunk_ = 0;
+
+  Path mult_path_ = Path::Own, multT_path_ = Path::Own;
+  // subspace tree: its tables (grid point per entry, -1 where none), and per
+  // precision (index 0 FP64, 1 FP32) the programs of mult and multTranspose
+  int64_t tree_total_ = 0, tree_nodes_ = 0;
+  int tree_depth_ = 0;
+  void* tree_ti_ = nullptr;  size_t tree_ti_cap_ = 0;
+  TreePlan tree_mult_[2], tree_multT_[2];
+  // boxes of a few data groups ([n][D][2]), to estimate what culling leaves
+  std::vector<double> probe_boxes_;
 
   // scratch
   void* A_ = nullptr;     size_t A_cap_ = 0;      // alpha*scale in compute type

@@ -48,9 +48,14 @@
 #include <sstream>
 
 #include "meval_kernels.hpp"
+#include "tree_device.hpp"
 
 namespace sgpp_hip {
 
+namespace {
+// data groups whose boxes estimate what culling leaves
+constexpr size_t kProbeGroups = 16;
+}  // namespace
 
 // Morton order of n points in [0,1]^d (row-major): b = min(16, 64/d) bits
 // per coordinate, interleaved from the top bit; ties keep the input order.
@@ -223,6 +228,19 @@ DeviceMultiEval::DeviceMultiEval(const double* data, size_t M, size_t dim, Basis
   check_hip(hipMemcpy(dperm_, dperm.data(), M_ * sizeof(int32_t), hipMemcpyHostToDevice),
             "upload data order");
   const bool templ = D_ <= static_cast<size_t>(kMaxTemplD);
+  if (templ && algorithm_ == Algorithm::Streaming) {
+    const int dim_i = static_cast<int>(D_);
+    const size_t group = 64 * static_cast<size_t>(serves(Precision::FP32) ? mult_k_rt<float>(dim_i)
+                                                                          : mult_k_rt<double>(dim_i));
+    const size_t ng = (M_ + group - 1) / group, n = std::min(kProbeGroups, ng);
+    probe_boxes_.resize(n * D_ * 2);
+    for (size_t p = 0; p < n; ++p)
+      for (size_t d = 0; d < D_; ++d) {
+        const double* col = soa.data() + d * Mpad_ + (ng * p / n) * group;
+        probe_boxes_[(p * D_ + d) * 2] = *std::min_element(col, col + group);
+        probe_boxes_[(p * D_ + d) * 2 + 1] = *std::max_element(col, col + group);
+      }
+  }
   if (serves(Precision::FP64)) {
     check_hip(hipMalloc(&X64_, soa.size() * sizeof(double)), "hipMalloc(X64)");
     check_hip(hipMemcpy(X64_, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice),
@@ -273,9 +291,12 @@ DeviceMultiEval::~DeviceMultiEval() {
   void* bufs[] = {X64_,   X32_,   WB64_,  WB32_,  LI64_,    LI32_,   TB64_,
                   TB32_,  scale_, perm_,  pm_,    dperm_,   A_,      Y_,
                   part_,  hin_,   hout_,  sub_desc_, sub_ti_, sub_te_, sub_tw_,
-                  sub_chunk_};
+                  sub_chunk_, tree_ti_};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  for (TreePlan* p : {&tree_mult_[0], &tree_mult_[1], &tree_multT_[0], &tree_multT_[1]})
+    for (void* b : {p->recs, p->chunks, p->groups})
+      if (b) (void)hipFree(b);
   for (auto* pool : {&tm_mult_, &tm_multT_})
     for (auto& e : *pool) {
       (void)hipEventDestroy(e.a);
@@ -316,6 +337,11 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   }
   std::vector<double> li0, sc0;
   encode_grid(basis_, D_, N, level, index, li0, sc0);
+  N_ = N;
+  Npad_ = ((N + kGridPad - 1) / kGridPad) * kGridPad;
+  TreeGrid tg;
+  if (set_paths(build_tree_grid(D_, N, level, index, true, tg) ? &tg : nullptr, li0, pmask))
+    return;
   // storage order: by the set of non-constant dimensions, then by the Morton
   // code of the support's centre, so that a 64-point tile holds points with
   // the same dimensions in a small region
@@ -383,6 +409,54 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
       choose_mult_order<float>(static_cast<const float*>(X32_), static_cast<const float*>(LI32_),
                                static_cast<const float*>(TB32_));
   }
+}
+
+// The walk of the subspace tree costs about kTreeCost operations per node and
+// data point whatever the data; the culled kernels two per evaluated dimension
+// and 2.5 more per grid point that a data group's box meets, estimated on a few
+// groups and grid points: on a d=8 grid of level 6 67 per node (FP32 mult 1,028
+// to 278 us), on an adaptive d=10 one 7 in FP64 (start 378 us, 280 us walked).
+constexpr double kTreeCost = 8.0;
+constexpr size_t kProbePoints = 16384;
+// multTranspose of the tree adds to LDS per node: it gains over the culled
+// kernel where launches count (1.3e6 nodes times data points, d=5, both products:
+// 329 to 60 us), not on a d=8 grid of level 6 (1,297 to 1,653 us).
+constexpr double kTreeMultTWork = 1e7;
+
+// Chooses the kernels of each direction (Path) and lays the grid out for them;
+// false if a direction is left to those of the instance's algorithm.
+bool DeviceMultiEval::set_paths(const TreeGrid* tree, const std::vector<double>& li,
+                                const std::vector<uint32_t>& pmask) {
+  mult_path_ = multT_path_ = Path::Own;
+  const double work = tree ? static_cast<double>(tree->node.size()) * static_cast<double>(M_) : 0.0;
+  const bool small = D_ > static_cast<size_t>(kMaxTemplD) || work <= kTreeMultTWork;
+  if (tree && (algorithm_ == Algorithm::Subspace || tree_pays(*tree, li, pmask)) &&
+      set_tree(*tree, small)) {
+    mult_path_ = Path::Tree;
+    if (small) multT_path_ = Path::Tree;
+  }
+  return mult_path_ != Path::Own && multT_path_ != Path::Own;
+}
+
+bool DeviceMultiEval::tree_pays(const TreeGrid& g, const std::vector<double>& li,
+                                const std::vector<uint32_t>& pmask) const {
+  if (D_ > static_cast<size_t>(kMaxTemplD)) return true;
+  const size_t N = pmask.size(), step = (N + kProbePoints - 1) / kProbePoints;
+  const size_t n = probe_boxes_.size() / (D_ * 2);
+  double cost = 0.0;
+  for (size_t p = 0; p < n; ++p) {
+    const double* box = &probe_boxes_[p * D_ * 2];
+    for (size_t j = 0; j < N; j += step) {
+      const double* row = &li[j * D_ * 2];
+      bool hit = true;
+      for (size_t d = 0; d < D_ && hit; ++d)
+        hit = row[2 * d] * box[2 * d + 1] - row[2 * d + 1] >= -1.0 &&
+              row[2 * d] * box[2 * d] - row[2 * d + 1] <= 1.0;
+      if (hit) cost += 2.0 * __builtin_popcount(pmask[j]) + 2.5;
+    }
+  }
+  cost *= static_cast<double>(step) / static_cast<double>(n);
+  return kTreeCost * static_cast<double>(g.node.size()) < cost;
 }
 
 // Block order of the templated mult and multTranspose kernels (the same
@@ -454,6 +528,17 @@ void DeviceMultiEval::choose_mult_order(const T* X, const T* LI, const float* TB
 void DeviceMultiEval::record_start() { check_hip(hipEventRecord(ev0_, stream_), "hipEventRecord"); }
 void DeviceMultiEval::record_stop() { check_hip(hipEventRecord(ev1_, stream_), "hipEventRecord"); }
 
+void DeviceMultiEval::check_scratch(const MultScratch& ext, size_t value_bytes) const {
+  const size_t a_bytes = (Npad_ * value_bytes + 255) / 256 * 256;
+  if (a_bytes + Mpad_ * sizeof(double) > ext.bytes) {
+    std::ostringstream os;
+    os << "input too large for the fixed scratch: " << N_ << " grid points and " << M_
+       << " data points need " << (a_bytes + Mpad_ * sizeof(double))
+       << " bytes at one grid chunk, the scratch holds " << ext.bytes;
+    throw input_error(os.str());
+  }
+}
+
 template <typename T>
 void DeviceMultiEval::run_mult(const T* X, const T* LI, const float* TB, const double* d_alpha,
                                double* d_result, hipEvent_t* tev, const MultScratch* ext) {
@@ -462,13 +547,7 @@ void DeviceMultiEval::run_mult(const T* X, const T* LI, const float* TB, const d
   const size_t a_bytes = (Npad_ * sizeof(T) + 255) / 256 * 256;
   void* A = nullptr;
   if (ext) {
-    if (a_bytes + Mpad_ * sizeof(double) > ext->bytes) {
-      std::ostringstream os;
-      os << "input too large for the fixed scratch: " << N_ << " grid points and " << M_
-         << " data points need " << (a_bytes + Mpad_ * sizeof(double))
-         << " bytes at one grid chunk, the scratch holds " << ext->bytes;
-      throw input_error(os.str());
-    }
+    check_scratch(*ext, sizeof(T));
     A = ext->base;
   } else {
     ensure(&A_, &A_cap_, Npad_ * sizeof(T));
@@ -604,7 +683,11 @@ void DeviceMultiEval::mult_device(const double* d_alpha, double* d_result, Preci
   EventPair* tp = timing_on_ ? next_timer(tm_mult_, used_mult_) : nullptr;
   hipEvent_t tev[2] = {tp ? tp->a : nullptr, tp ? tp->b : nullptr};
   record_start();
-  if (algorithm_ == Algorithm::Subspace)
+  if (mult_path_ == Path::Tree && p == Precision::FP64)
+    run_tree_mult<double>(d_alpha, d_result, tp ? tev : nullptr);
+  else if (mult_path_ == Path::Tree)
+    run_tree_mult<float>(d_alpha, d_result, tp ? tev : nullptr);
+  else if (algorithm_ == Algorithm::Subspace)
     run_subspace_mult(d_alpha, d_result, tp ? tev : nullptr);
   else if (p == Precision::FP64)
     run_mult<double>(static_cast<const double*>(X64_), static_cast<const double*>(LI64_),
@@ -650,7 +733,11 @@ void DeviceMultiEval::mult_device_noalloc(const double* d_alpha, double* d_resul
   const MultScratch sc{device_scratch(device_), kNoAllocScratchBytes};
   check_hip(hipSetDevice(device_), "hipSetDevice");
   record_start();
-  if (p == Precision::FP64)
+  if (mult_path_ == Path::Tree && p == Precision::FP64)
+    run_tree_mult<double>(d_alpha, d_result, nullptr, &sc);
+  else if (mult_path_ == Path::Tree)
+    run_tree_mult<float>(d_alpha, d_result, nullptr, &sc);
+  else if (p == Precision::FP64)
     run_mult<double>(static_cast<const double*>(X64_), static_cast<const double*>(LI64_),
                      static_cast<const float*>(TB64_), d_alpha, d_result, nullptr, &sc);
   else
@@ -666,7 +753,11 @@ void DeviceMultiEval::mult_transpose_device(const double* d_y, double* d_result,
   EventPair* tp = timing_on_ ? next_timer(tm_multT_, used_multT_) : nullptr;
   hipEvent_t tev[2] = {tp ? tp->a : nullptr, tp ? tp->b : nullptr};
   record_start();
-  if (algorithm_ == Algorithm::Subspace)
+  if (multT_path_ == Path::Tree && p == Precision::FP64)
+    run_tree_multT<double>(d_y, d_result, tp ? tev : nullptr);
+  else if (multT_path_ == Path::Tree)
+    run_tree_multT<float>(d_y, d_result, tp ? tev : nullptr);
+  else if (algorithm_ == Algorithm::Subspace)
     run_subspace_multT(d_y, d_result, tp ? tev : nullptr);
   else if (p == Precision::FP64)
     run_multT<double>(static_cast<const double*>(X64_), static_cast<const double*>(LI64_),
@@ -686,6 +777,13 @@ void DeviceMultiEval::count_work(Precision p, uint64_t out[4]) {
     out[1] = out[3] = static_cast<uint64_t>(Mpad_) * static_cast<uint64_t>(nsub_);
     out[0] = static_cast<uint64_t>(Mpad_) * sub_recompute_;
     out[2] = static_cast<uint64_t>(Mpad_) * sub_recompute_t_;
+    return;
+  }
+  // the tree: one factor and one pair per data row and node
+  const uint64_t walked = static_cast<uint64_t>(M_) * static_cast<uint64_t>(tree_nodes_);
+  if (mult_path_ != Path::Own && multT_path_ != Path::Own) {
+    out[0] = out[1] = walked;
+    out[2] = out[3] = walked;
     return;
   }
   check_hip(hipSetDevice(device_), "hipSetDevice");
@@ -717,6 +815,8 @@ void DeviceMultiEval::count_work(Precision p, uint64_t out[4]) {
   }
   timing_on_ = timing;
   check_hip(hipFree(dcnt), "hipFree(counters)");
+  if (mult_path_ != Path::Own) out[0] = out[1] = walked;
+  if (multT_path_ != Path::Own) out[2] = out[3] = walked;
   if (D_ > static_cast<size_t>(kMaxTemplD)) {
     // the generic kernels evaluate every pair of the padded arrays in every dimension
     const uint64_t jend = static_cast<uint64_t>(ceil_div(N_, kTG)) * kTG;

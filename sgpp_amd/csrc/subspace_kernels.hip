@@ -45,6 +45,7 @@
 #include "cull_device.hpp"
 #include "meval_device.hpp"
 #include "subspace_device.hpp"
+#include "tree_device.hpp"
 
 namespace sgpp_hip {
 
@@ -334,6 +335,37 @@ SubspaceLayout build_subspace_layout(size_t D, size_t N, const uint32_t* level,
 
 void DeviceMultiEval::set_grid_subspace(const uint32_t* level, const uint32_t* index, size_t N) {
   check_hip(hipSetDevice(device_), "hipSetDevice");
+  TreeGrid tg;
+  build_tree_grid(D_, N, level, index, false, tg);
+  // the subspaces in lexicographic order: the dimensions evaluated per data row
+  // (those shared with the previous one left out), and the chunks of this
+  // algorithm's multTranspose
+  std::vector<const uint8_t*> lv(tg.node.size());
+  for (size_t s = 0; s < lv.size(); ++s) lv[s] = &tg.level[s * D_];
+  std::sort(lv.begin(), lv.end(), [&](const uint8_t* a, const uint8_t* b) {
+    return std::lexicographical_compare(a, a + D_, b, b + D_);
+  });
+  uint64_t steps = 0;
+  int64_t nchunk = 0, fill = kSubLds;
+  for (size_t s = 0; s < lv.size(); ++s) {
+    int bits = 0;
+    for (size_t d = 0; d < D_; ++d) bits += lv[s][d] - 1;
+    const int64_t n = int64_t(1) << bits;
+    if (fill + n > kSubLds) ++nchunk;
+    fill = n > kSubLds ? kSubLds : (fill + n > kSubLds ? n : fill + n);
+    size_t d = 0;
+    while (s && lv[s][d] == lv[s - 1][d]) ++d;
+    for (; d < D_; ++d) steps += !(basis_ == Basis::ModLinear && lv[s][d] == 1);
+  }
+  if (nchunk > 65535) throw input_error("too many subspace chunks for one launch");
+  if (set_paths(&tg, {}, {})) {
+    N_ = N;
+    Npad_ = N;
+    nsub_ = static_cast<int>(tg.node.size());
+    ntable_ = tg.total;
+    sub_recompute_ = sub_recompute_t_ = steps;
+    return;
+  }
   SubspaceLayout lay = build_subspace_layout(D_, N, level, index);
   std::vector<SubspaceDesc>& desc = lay.desc;
   const int64_t total = lay.total;

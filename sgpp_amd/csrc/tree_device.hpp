@@ -1,0 +1,148 @@
+// The subspace tree: grids evaluated subspace by subspace, one
+// one-dimensional factor per (data point, subspace). Data structures shared by
+// the kernels (tree_kernels.hpp), their instantiations and the runtime
+// (tree_runtime.hip).
+//
+// In a subspace W_l (level vector l) the supports of the basis functions tile
+// [0,1]^d, so a data point lies in the support of exactly one of them (after
+// the reference's SubspaceLinear operator,
+// OperationMultipleEvalSubspaceCombined.hpp:92-204). The level vectors form a
+// tree: the parent of l is l with its last level above 1 set to 1, so a
+// subspace's basis value is its parent's times ONE factor, and its table
+// position is its parent's extended by one cell number. The subspaces are kept
+// in depth-first order, a parent's children by dimension, then level.
+//
+// A program is the tree's nodes as 16-byte records in that order; a wave walks
+// it with one or more data points per lane, the parents' products and table
+// positions in registers, one set per depth.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+#include "meval_device.hpp"
+#include "subspace_device.hpp"
+
+namespace sgpp_hip {
+
+// Levels above 1 of one level vector at most (the register sets of a walk);
+// deeper grids are left to the other kernels.
+constexpr int kTreeMaxDepth = 12;
+
+// threads of a mult block (four waves share one chunk's tables)
+constexpr int kTreeBlock = 256;
+
+// ctl of a record
+constexpr uint32_t kTreeShiftMask = 31u;    // 33 - level
+constexpr int kTreeDimShift = 8;            // 6 bits: the dimension
+constexpr uint32_t kTreeRun = 1u << 16;     // first of its (parent, dimension): fetch x, the parent's product
+constexpr uint32_t kTreeTable = 1u << 17;   // the subspace has grid points (absent parents are walked without)
+constexpr uint32_t kTreePush = 1u << 18;    // children follow
+constexpr uint32_t kTreeLast = 1u << 19;    // last of its parent's children
+constexpr uint32_t kTreeFlush = 1u << 20;   // add the FP32 sums to the FP64 ones
+
+constexpr uint32_t kTreePart = 1u << 21;    // (without kTreeTable) part of a table: see TreeChunk
+
+struct alignas(16) TreeRec {
+  uint32_t off;    // byte offset of the subspace's table in the chunk's LDS image
+  uint32_t ctl;
+  uint32_t scale;  // 2^(level - 1): the float's bits, or the double's upper word
+  uint32_t from;   // a run's first record: the dimensions [from, dim) to pass (Linear)
+};
+static_assert(sizeof(TreeRec) == 16, "one record is 16 bytes");
+
+// A run of consecutive subspaces whose tables fit the LDS image: records
+// [rec0, rec0 + nrec), table entries [off0, off0 + n). root: the chunk begins
+// with the subspace of level 1 in every dimension (one entry, the first).
+// part: one subspace whose table exceeds the image; the chunk holds its
+// positions [part0, part0 + n).
+struct alignas(16) TreeChunk {
+  int rec0, nrec;
+  int n, part0;
+  long long off0;
+  int root, part;
+};
+static_assert(sizeof(TreeChunk) == 32, "one chunk is 32 bytes");
+
+// A grid's subspaces in walking order, and their tables.
+struct TreeGrid {
+  struct Node {
+    int depth;             // levels above 1
+    int64_t off;           // table offset
+    int bits;              // table entries: 2^bits
+  };
+  size_t D = 0;
+  std::vector<uint8_t> level;  // [nodes][D]
+  std::vector<Node> node;
+  std::vector<int32_t> ti;     // grid point of a table entry, or -1
+  int64_t total = 0;           // table entries
+  int depth = 0;               // of the deepest node
+  bool repeated = false;       // a grid point occurs twice (a table holds it once)
+};
+// Sorts the points by subspace and builds the tables. Throws input_error
+// for points outside a no-boundary grid and for tables beyond
+// subspace_table_limit(N) or 2^30 cells in one subspace; with quiet it returns
+// false for the latter two instead.
+bool build_tree_grid(size_t D, size_t N, const uint32_t* level, const uint32_t* index,
+                     bool quiet, TreeGrid& g);
+
+// Programs of a grid: groups of chunks of at most cap table entries and
+// max_nodes nodes; the groups have about equal numbers of nodes.
+struct TreeProgram {
+  std::vector<TreeRec> recs;
+  std::vector<TreeChunk> chunks;
+  std::vector<int> groups;
+  int max_entries = 0;
+};
+TreeProgram build_tree_program(const TreeGrid& g, int ngroups, int64_t cap, int64_t max_nodes,
+                               int entry_bytes, bool fp32);
+
+struct TreeMultArgs {
+  const void* X;  // [D][ldx], stored order
+  int64_t ldx, M;
+  int D;
+  const TreeRec* recs;
+  const TreeChunk* chunks;
+  const int* groups;  // chunk group g: chunks [groups[g], groups[g + 1])
+  int ngroups, gper;  // groups, and groups per block (blockIdx.y)
+  const void* W;      // weights in table order and compute type, or null:
+  const double* alpha;  // gathered from here through ti
+  const int32_t* ti;
+  double* part;  // [gridDim.y][ldx], or null: results to out[dperm[m]]
+  double* out;
+  const int32_t* dperm;
+  int zero_off;  // byte offset of an LDS zero (rows outside a part)
+};
+
+struct TreeMultTArgs {
+  const void* X;
+  int64_t ldx;
+  int D;
+  const void* Y;  // [ldx] stored order, compute type, 0 past the data
+  const TreeRec* recs;
+  const TreeChunk* chunks;
+  int64_t seg, mend;  // rows per segment (blockIdx.y), end of the rows
+  double* part;       // [segments][ntable]
+  int64_t ntable;
+};
+
+// Launchers of one compute type and basis. wide: several data points per
+// lane; D: dimensions, depth: of the grid's tree. rows(): data points per
+// wave.
+struct TreeLaunch {
+  int k = 1;
+  void (*mult)(const TreeMultArgs&, dim3 grid, unsigned block, unsigned lds, hipStream_t s) = nullptr;
+  int kt = 1;
+  void (*multT)(const TreeMultTArgs&, dim3 grid, unsigned lds, hipStream_t s) = nullptr;
+};
+template <typename T, bool kMod>
+TreeLaunch tree_launch(int D, int depth, bool wide);
+extern template TreeLaunch tree_launch<float, false>(int, int, bool);
+extern template TreeLaunch tree_launch<float, true>(int, int, bool);
+extern template TreeLaunch tree_launch<double, false>(int, int, bool);
+extern template TreeLaunch tree_launch<double, true>(int, int, bool);
+
+}  // namespace sgpp_hip

@@ -1,0 +1,480 @@
+// Runtime of the subspace-tree algorithm (tree_device.hpp): grids and
+// programs on the host, launch shapes, the small kernels around the walks.
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <numeric>
+
+#include "parts_device.hpp"
+#include "tree_device.hpp"
+
+namespace sgpp_hip {
+
+namespace {
+
+// W[e] = alpha[ti[e]] in the compute type (0 where the entry has no grid point)
+template <typename T>
+__global__ void tree_weights_kernel(const double* __restrict__ alpha,
+                                    const int32_t* __restrict__ ti, T* __restrict__ W, int64_t n) {
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e < n) W[e] = ti[e] >= 0 ? static_cast<T>(alpha[ti[e]]) : T(0);
+}
+
+}  // namespace
+
+bool build_tree_grid(size_t D, size_t N, const uint32_t* level, const uint32_t* index,
+                     bool quiet, TreeGrid& g) {
+  g = TreeGrid();
+  g.D = D;
+  for (size_t e = 0; e < N * D; ++e) {
+    const uint32_t l = level[e], i = index[e];
+    if (l < 1 || l > 30 || (i & 1u) == 0 || i >= (1u << l))
+      throw input_error("invalid grid point (level/index out of range for a no-boundary grid)");
+  }
+  // points by subspace in depth-first order: the steps (dimension, level above
+  // 1) compare one by one, a parent before its children. As numbers per
+  // dimension: the level, or for level 1 a value above all levels where
+  // another step follows (its dimension is larger) and 0 where none does.
+  // 5 bits each: two words hold 24 dimensions.
+  std::vector<uint32_t> order(N);
+  std::iota(order.begin(), order.end(), 0u);
+  if (D <= 24) {
+    struct Key {
+      uint64_t a, b;
+      uint32_t j;
+    };
+    std::vector<Key> key(N);
+    for (size_t j = 0; j < N; ++j) {
+      uint64_t w[2] = {0, 0};
+      bool later = false;
+      for (size_t d = D; d-- > 0;) {
+        const uint64_t l = level[j * D + d];
+        w[d / 12] |= (l > 1 ? l : (later ? 31u : 0u)) << (5 * (11 - d % 12));
+        later |= l > 1;
+      }
+      key[j] = Key{w[0], w[1], static_cast<uint32_t>(j)};
+    }
+    std::sort(key.begin(), key.end(), [](const Key& x, const Key& y) {
+      return x.a != y.a ? x.a < y.a : (x.b != y.b ? x.b < y.b : x.j < y.j);
+    });
+    for (size_t s = 0; s < N; ++s) order[s] = key[s].j;
+  } else {
+    auto later = [&](const uint32_t* p, size_t d) {
+      while (++d < D)
+        if (p[d] > 1) return true;
+      return false;
+    };
+    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
+      const uint32_t *p = level + x * D, *q = level + y * D;
+      for (size_t d = 0; d < D; ++d)
+        if (p[d] != q[d]) {
+          if (p[d] == 1) return !later(p, d);
+          if (q[d] == 1) return later(q, d);
+          return p[d] < q[d];
+        }
+      return x < y;
+    });
+  }
+  const int64_t limit = subspace_table_limit(N);
+  for (size_t s = 0; s < N; ++s) {
+    const uint32_t* lv = level + static_cast<size_t>(order[s]) * D;
+    if (s && std::memcmp(level + static_cast<size_t>(order[s - 1]) * D, lv, D * sizeof(uint32_t)) == 0)
+      continue;
+    TreeGrid::Node n{0, g.total, 0};
+    int64_t bits = 0;
+    for (size_t d = 0; d < D; ++d) {
+      n.depth += lv[d] > 1;
+      bits += lv[d] - 1;
+      g.level.push_back(static_cast<uint8_t>(lv[d]));
+    }
+    if (bits > 30) {
+      if (quiet) return false;
+      throw input_error("a subspace's index table would exceed 2^30 entries");
+    }
+    n.bits = static_cast<int>(bits);
+    g.total += int64_t(1) << bits;
+    if (g.total > limit) {
+      if (quiet) return false;
+      throw input_error("the subspace index tables of this grid would hold more than 64 entries "
+                        "per grid point");
+    }
+    g.depth = std::max(g.depth, n.depth);
+    g.node.push_back(n);
+  }
+  g.ti.assign(static_cast<size_t>(g.total), -1);
+  size_t at = 0;
+  for (size_t s = 0; s < N; ++s) {
+    const uint32_t* lv = level + static_cast<size_t>(order[s]) * D;
+    const uint32_t* ix = index + static_cast<size_t>(order[s]) * D;
+    if (s) {
+      const uint32_t* before = level + static_cast<size_t>(order[s - 1]) * D;
+      if (std::memcmp(before, lv, D * sizeof(uint32_t)) != 0) ++at;
+    }
+    int64_t flat = 0;
+    for (size_t d = 0; d < D; ++d) flat = (flat << (lv[d] - 1)) + (ix[d] >> 1);
+    int32_t& entry = g.ti[static_cast<size_t>(g.node[at].off + flat)];
+    g.repeated |= entry >= 0;
+    entry = static_cast<int32_t>(order[s]);
+  }
+  return true;
+}
+
+namespace {
+
+// nodes between two additions of the FP32 sums to the FP64 ones
+constexpr int kFlushNodes = 64;
+
+struct Step {
+  int dim, level;
+};
+
+// Appends the program of nodes [a, b) (b > a; the root, where it is one of
+// them, is not a record). Table offsets are relative to off0; no_table: the
+// nodes' tables are left to the caller's part chunk (kTreePart).
+void append_program(const TreeGrid& g, size_t a, size_t b, int64_t off0, int entry_bytes, bool fp32,
+                    bool part, TreeProgram& p) {  // (depth at most kTreeMaxDepth)
+  struct Emit {
+    int depth, dim, level;
+    uint32_t off, flags;
+  };
+  std::vector<Emit> out;
+  std::vector<Step> path, steps;
+  int since = 0;
+  for (size_t s = a; s < b; ++s) {
+    const uint8_t* lv = &g.level[s * g.D];
+    steps.clear();
+    for (size_t d = 0; d < g.D; ++d)
+      if (lv[d] > 1) steps.push_back(Step{static_cast<int>(d), lv[d]});
+    if (steps.empty()) continue;  // the root
+    size_t same = 0;
+    while (same < path.size() && same < steps.size() && path[same].dim == steps[same].dim &&
+           path[same].level == steps[same].level)
+      ++same;
+    // ancestors that are not on the path (at a chunk's start, or not in the
+    // grid) are walked without a table
+    for (size_t q = same; q + 1 < steps.size(); ++q)
+      out.push_back(Emit{static_cast<int>(q), steps[q].dim, steps[q].level, 0u, 0u});
+    uint32_t flags = part ? kTreePart : kTreeTable;
+    if (fp32 && ++since == kFlushNodes) {
+      flags |= kTreeFlush;
+      since = 0;
+    }
+    out.push_back(Emit{static_cast<int>(steps.size()) - 1, steps.back().dim, steps.back().level,
+                       static_cast<uint32_t>((part ? -off0 : g.node[s].off - off0) * entry_bytes),
+                       flags});
+    path = steps;
+  }
+  // the dimensions that the product at each depth covers
+  int covered[kTreeMaxDepth + 2] = {};
+  for (size_t i = 0; i < out.size(); ++i) {
+    Emit& e = out[i];
+    if (i + 1 < out.size() && out[i + 1].depth == e.depth + 1) e.flags |= kTreePush;
+    const bool follows = i > 0 && out[i - 1].depth == e.depth && out[i - 1].dim == e.dim &&
+                         !(out[i - 1].flags & kTreePush);
+    if (!follows) e.flags |= kTreeRun;
+    size_t q = i + 1;
+    while (q < out.size() && out[q].depth > e.depth) ++q;
+    if (q == out.size() || out[q].depth < e.depth) e.flags |= kTreeLast;
+    TreeRec r{};
+    r.off = e.off;
+    r.ctl = static_cast<uint32_t>(33 - e.level) | (static_cast<uint32_t>(e.dim) << kTreeDimShift) |
+            e.flags;
+    r.from = static_cast<uint32_t>(covered[e.depth]);
+    covered[e.depth] = e.dim;
+    covered[e.depth + 1] = e.dim + 1;
+    r.scale = fp32 ? static_cast<uint32_t>(127 + e.level - 1) << 23
+                   : static_cast<uint32_t>(1023 + e.level - 1) << 20;
+    p.recs.push_back(r);
+  }
+}
+
+}  // namespace
+
+TreeProgram build_tree_program(const TreeGrid& g, int ngroups, int64_t cap, int64_t max_nodes,
+                               int entry_bytes, bool fp32) {
+  TreeProgram p;
+  const size_t n = g.node.size();
+  ngroups = static_cast<int>(std::max<size_t>(1, std::min<size_t>(ngroups, n)));
+  for (int q = 0; q < ngroups; ++q) {
+    const size_t g0 = n * q / ngroups, g1 = n * (q + 1) / ngroups;
+    p.groups.push_back(static_cast<int>(p.chunks.size()));
+    for (size_t a = g0; a < g1;) {
+      const int64_t size = int64_t(1) << g.node[a].bits;
+      if (size > cap) {
+        // one subspace in parts of cap positions
+        for (int64_t s = 0; s < size; s += cap) {
+          TreeChunk c{};
+          c.rec0 = static_cast<int>(p.recs.size());
+          append_program(g, a, a + 1, s, entry_bytes, fp32, true, p);
+          c.nrec = static_cast<int>(p.recs.size()) - c.rec0;
+          c.n = static_cast<int>(std::min(cap, size - s));
+          c.part0 = static_cast<int>(s);
+          c.off0 = g.node[a].off + s;
+          p.max_entries = std::max(p.max_entries, c.n);
+          p.chunks.push_back(c);
+        }
+        ++a;
+        continue;
+      }
+      size_t b = a;
+      const int64_t off0 = g.node[a].off;
+      int64_t entries = 0;
+      while (b < g1 && static_cast<int64_t>(b - a) < max_nodes) {
+        const int64_t more = int64_t(1) << g.node[b].bits;
+        if (entries + more > cap) break;
+        entries += more;
+        ++b;
+      }
+      TreeChunk c{};
+      c.rec0 = static_cast<int>(p.recs.size());
+      append_program(g, a, b, off0, entry_bytes, fp32, false, p);
+      c.nrec = static_cast<int>(p.recs.size()) - c.rec0;
+      c.n = static_cast<int>(entries);
+      c.off0 = off0;
+      c.root = g.node[a].depth == 0;
+      p.max_entries = std::max(p.max_entries, c.n);
+      p.chunks.push_back(c);
+      a = b;
+    }
+  }
+  p.groups.push_back(static_cast<int>(p.chunks.size()));
+  p.recs.push_back(TreeRec{});  // read ahead of the last record
+  return p;
+}
+
+// ----------------------------------------------------------------- shapes
+
+namespace {
+
+// LDS of a mult block and of a multTranspose wave: 40 KiB and 10 KiB let the
+// registers, not the LDS, bound the waves in flight (16 per CU, 12 for Linear)
+constexpr int kMultLds = 40 << 10;
+constexpr int kMultTEntries = 1280;
+// nodes per chunk group (mult) or chunk (multTranspose) at least, so that a
+// wave's start is small against its walk
+constexpr int kMinNodes = 8;
+constexpr int64_t kTreePartialBudget = int64_t(2048) << 20;
+
+}  // namespace
+
+void DeviceMultiEval::upload_tree(const TreeProgram& p, TreePlan& plan, int entry_bytes) {
+  plan.nchunks = static_cast<int>(p.chunks.size());
+  plan.ngroups = static_cast<int>(p.groups.size()) - 1;
+  plan.lds = (p.max_entries * entry_bytes + 15) / 16 * 16;
+  ensure(&plan.recs, &plan.recs_cap, p.recs.size() * sizeof(TreeRec));
+  check_hip(hipMemcpy(plan.recs, p.recs.data(), p.recs.size() * sizeof(TreeRec),
+                      hipMemcpyHostToDevice),
+            "upload tree records");
+  ensure(&plan.chunks, &plan.chunks_cap, p.chunks.size() * sizeof(TreeChunk));
+  check_hip(hipMemcpy(plan.chunks, p.chunks.data(), p.chunks.size() * sizeof(TreeChunk),
+                      hipMemcpyHostToDevice),
+            "upload tree chunks");
+  ensure(&plan.groups, &plan.groups_cap, p.groups.size() * sizeof(int));
+  check_hip(hipMemcpy(plan.groups, p.groups.data(), p.groups.size() * sizeof(int),
+                      hipMemcpyHostToDevice),
+            "upload tree groups");
+}
+
+template <typename T>
+void DeviceMultiEval::set_tree_plans(const TreeGrid& g, bool multT) {
+  const int ix = sizeof(T) == sizeof(double) ? 0 : 1;
+  const bool mod = basis_ == Basis::ModLinear;
+  const int64_t nodes = static_cast<int64_t>(g.node.size());
+  const int64_t M = static_cast<int64_t>(M_);
+  const int waves_cu = mod ? 16 : 12;
+  const int64_t slots = static_cast<int64_t>(num_cus_) * waves_cu;
+  auto launch = [&](bool wide) {
+    return mod ? tree_launch<T, true>(static_cast<int>(D_), g.depth, wide)
+               : tree_launch<T, false>(static_cast<int>(D_), g.depth, wide);
+  };
+  // several points per lane where that leaves every wave slot a walk of kMinNodes
+  TreeLaunch l = launch(true);
+  const bool wide = M * nodes >= slots * 64 * l.k * kMinNodes;
+  l = launch(wide);
+  // mult: chunk groups so that the blocks fill the device evenly
+  TreePlan& pm = tree_mult_[ix];
+  pm.wide = wide;
+  const int64_t rb = (M + kTreeBlock * l.k - 1) / (kTreeBlock * l.k);
+  const int64_t bslots = slots / (kTreeBlock / 64);
+  int64_t G = cfg_.mult_grid_chunks;
+  if (G <= 0) {
+    const int64_t gmax = std::max<int64_t>(1, std::min<int64_t>(64, nodes / kMinNodes));
+    double best = 0.0;
+    for (int64_t q = 1; q <= gmax; ++q) {
+      // nanoseconds per data point: the walk with the last round's idle
+      // blocks, the FP64 partials written and read
+      const double b = static_cast<double>(rb * q);
+      const double walk = 2e-4 * static_cast<double>(nodes) *
+                          std::ceil(b / static_cast<double>(bslots)) * static_cast<double>(bslots) / b;
+      const double t = walk + (q > 1 ? 0.005 * static_cast<double>(q) : 0.0);
+      if (q == 1 || t < best * 0.98) {
+        best = t;
+        G = q;
+      }
+    }
+    G = std::min<int64_t>(G, std::max<int64_t>(1, kTreePartialBudget / (Mpad_ * sizeof(double))));
+  }
+  upload_tree(build_tree_program(g, static_cast<int>(std::min<int64_t>(G, nodes)),
+                                 (kMultLds - 16) / static_cast<int64_t>(sizeof(T)), nodes,
+                                 static_cast<int>(sizeof(T)), sizeof(T) == 4),
+              pm, static_cast<int>(sizeof(T)));
+  if (!multT) return;
+  // multTranspose: chunks, each a wave per data segment
+  TreePlan& pt = tree_multT_[ix];
+  pt.wide = wide;
+  const int64_t batches = (M + 64 * l.kt - 1) / (64 * l.kt);
+  const int64_t per = std::max<int64_t>(kMinNodes, nodes * batches / slots);
+  upload_tree(build_tree_program(g, 1, kMultTEntries, per, 8, sizeof(T) == 4), pt, 8);
+}
+
+bool DeviceMultiEval::set_tree(const TreeGrid& g, bool multT) {
+  if (g.repeated || g.depth > kTreeMaxDepth || g.node.size() > (size_t(1) << 24)) return false;
+  check_hip(hipSetDevice(device_), "hipSetDevice");
+  check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+  ensure(&tree_ti_, &tree_ti_cap_, g.ti.size() * sizeof(int32_t));
+  check_hip(hipMemcpy(tree_ti_, g.ti.data(), g.ti.size() * sizeof(int32_t), hipMemcpyHostToDevice),
+            "upload tables");
+  tree_total_ = g.total;
+  tree_nodes_ = static_cast<int64_t>(g.node.size());
+  tree_depth_ = g.depth;
+  if (serves(Precision::FP64)) set_tree_plans<double>(g, multT);
+  if (serves(Precision::FP32)) set_tree_plans<float>(g, multT);
+  return true;
+}
+
+// ---------------------------------------------------------------- launches
+
+template <typename T>
+void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hipEvent_t* tev,
+                                    const MultScratch* ext) {
+  hipStream_t s = stream_;
+  const TreePlan& plan = tree_mult_[sizeof(T) == sizeof(double) ? 0 : 1];
+  const TreeLaunch l = basis_ == Basis::ModLinear
+                           ? tree_launch<T, true>(static_cast<int>(D_), tree_depth_, plan.wide)
+                           : tree_launch<T, false>(static_cast<int>(D_), tree_depth_, plan.wide);
+  const int64_t M = static_cast<int64_t>(M_);
+  const unsigned rb = blocks(M, kTreeBlock * l.k);
+  int G = plan.ngroups, gper = 1;
+  // weights in table order first, unless few blocks gather few of them
+  const size_t wbytes = (static_cast<size_t>(tree_total_) * sizeof(T) + 255) / 256 * 256;
+  bool weights = static_cast<int64_t>(rb) * tree_total_ > (int64_t(1) << 21);
+  double* P = nullptr;
+  T* W = nullptr;
+  if (ext) {
+    check_scratch(*ext, sizeof(T));
+    if (wbytes > ext->bytes) weights = false;
+    const size_t left = ext->bytes - (weights ? wbytes : 0);
+    const int64_t rows = static_cast<int64_t>(left / (Mpad_ * sizeof(double)));
+    if (rows < G) gper = rows > 1 ? static_cast<int>((G + rows - 1) / rows) : G;
+    if (weights) W = static_cast<T*>(ext->base);
+    P = reinterpret_cast<double*>(static_cast<unsigned char*>(ext->base) + (weights ? wbytes : 0));
+  } else if (weights) {
+    ensure(&A_, &A_cap_, wbytes);
+    W = static_cast<T*>(A_);
+  }
+  G = (G + gper - 1) / gper;
+  if (G > 1 && !ext) {
+    ensure(&part_, &part_cap_, static_cast<size_t>(G) * Mpad_ * sizeof(double));
+    P = static_cast<double*>(part_);
+  }
+  if (weights) {
+    clear_launch_error();
+    hipLaunchKernelGGL(tree_weights_kernel<T>, dim3(blocks(tree_total_, 256)), dim3(256), 0, s,
+                       d_alpha, static_cast<const int32_t*>(tree_ti_), W, tree_total_);
+    check_hip(hipGetLastError(), "tree weights");
+  }
+  TreeMultArgs a{};
+  a.X = sizeof(T) == sizeof(double) ? X64_ : X32_;
+  a.ldx = static_cast<int64_t>(Mpad_);
+  a.M = M;
+  a.D = static_cast<int>(D_);
+  a.recs = static_cast<const TreeRec*>(plan.recs);
+  a.chunks = static_cast<const TreeChunk*>(plan.chunks);
+  a.groups = static_cast<const int*>(plan.groups);
+  a.ngroups = plan.ngroups;
+  a.gper = gper;
+  a.W = W;
+  a.alpha = d_alpha;
+  a.ti = static_cast<const int32_t*>(tree_ti_);
+  a.part = G > 1 ? P : nullptr;
+  a.out = d_result;
+  a.dperm = static_cast<const int32_t*>(dperm_);
+  a.zero_off = plan.lds;
+  if (tev) check_hip(hipEventRecord(tev[0], s), "hipEventRecord");
+  l.mult(a, dim3(rb, static_cast<unsigned>(G)), kTreeBlock, static_cast<unsigned>(plan.lds) + 16, s);
+  check_hip(hipGetLastError(), "tree mult kernel");
+  if (tev) check_hip(hipEventRecord(tev[1], s), "hipEventRecord");
+  if (G > 1) {
+    clear_launch_error();
+    hipLaunchKernelGGL(reduce_rows_kernel, dim3(blocks(M, kCols)), dim3(kRows * kCols), 0, s, P,
+                       static_cast<int64_t>(Mpad_), G, static_cast<const int32_t*>(dperm_),
+                       static_cast<const double*>(nullptr), d_result, M);
+    check_hip(hipGetLastError(), "tree reduce (mult)");
+  }
+  last_G_ = G;
+}
+
+template <typename T>
+void DeviceMultiEval::run_tree_multT(const double* d_y, double* d_result, hipEvent_t* tev) {
+  hipStream_t s = stream_;
+  const TreePlan& plan = tree_multT_[sizeof(T) == sizeof(double) ? 0 : 1];
+  const TreeLaunch l = basis_ == Basis::ModLinear
+                           ? tree_launch<T, true>(static_cast<int>(D_), tree_depth_, plan.wide)
+                           : tree_launch<T, false>(static_cast<int>(D_), tree_depth_, plan.wide);
+  const int64_t M = static_cast<int64_t>(M_), rows = 64 * l.kt;
+  const int64_t batches = (M + rows - 1) / rows;
+  int64_t S = cfg_.multT_data_segs;
+  if (S <= 0) {
+    // two rounds of waves
+    const int waves_cu = basis_ == Basis::ModLinear ? 16 : 12;
+    const int64_t target = cfg_.target_blocks > 0 ? cfg_.target_blocks
+                                                  : 2 * static_cast<int64_t>(num_cus_) * waves_cu;
+    S = std::max<int64_t>(1, target / plan.nchunks);
+    S = std::min<int64_t>(S, std::max<int64_t>(1, kTreePartialBudget / (tree_total_ * 8)));
+  }
+  S = std::min<int64_t>({S, batches, 65535});
+  const int64_t seg = (batches + S - 1) / S * rows;
+  S = (batches * rows + seg - 1) / seg;
+  ensure(&Y_, &Y_cap_, Mpad_ * sizeof(T));
+  ensure(&part_, &part_cap_, static_cast<size_t>(S * tree_total_) * sizeof(double));
+  clear_launch_error();
+  hipLaunchKernelGGL(prep_rows_kernel<T>, dim3(blocks(Mpad_, 256)), dim3(256), 0, s, d_y,
+                     static_cast<const int32_t*>(dperm_), static_cast<T*>(Y_), M,
+                     static_cast<int64_t>(Mpad_));
+  check_hip(hipGetLastError(), "tree prep");
+  TreeMultTArgs a{};
+  a.X = sizeof(T) == sizeof(double) ? X64_ : X32_;
+  a.ldx = static_cast<int64_t>(Mpad_);
+  a.D = static_cast<int>(D_);
+  a.Y = Y_;
+  a.recs = static_cast<const TreeRec*>(plan.recs);
+  a.chunks = static_cast<const TreeChunk*>(plan.chunks);
+  a.seg = seg;
+  a.mend = batches * rows;
+  a.part = static_cast<double*>(part_);
+  a.ntable = tree_total_;
+  if (tev) check_hip(hipEventRecord(tev[0], s), "hipEventRecord");
+  l.multT(a, dim3(static_cast<unsigned>(plan.nchunks), static_cast<unsigned>(S)),
+          static_cast<unsigned>(plan.lds), s);
+  check_hip(hipGetLastError(), "tree multTranspose kernel");
+  if (tev) check_hip(hipEventRecord(tev[1], s), "hipEventRecord");
+  clear_launch_error();
+  hipLaunchKernelGGL(reduce_rows_kernel, dim3(blocks(tree_total_, kCols)), dim3(kRows * kCols), 0,
+                     s, static_cast<const double*>(part_), tree_total_, static_cast<int>(S),
+                     static_cast<const int32_t*>(tree_ti_),
+                     static_cast<const double*>(nullptr), d_result, tree_total_);
+  check_hip(hipGetLastError(), "tree reduce (multTranspose)");
+  last_S_ = static_cast<int>(S);
+}
+
+template void DeviceMultiEval::run_tree_mult<double>(const double*, double*, hipEvent_t*,
+                                                     const MultScratch*);
+template void DeviceMultiEval::run_tree_mult<float>(const double*, double*, hipEvent_t*,
+                                                    const MultScratch*);
+template void DeviceMultiEval::run_tree_multT<double>(const double*, double*, hipEvent_t*);
+template void DeviceMultiEval::run_tree_multT<float>(const double*, double*, hipEvent_t*);
+
+}  // namespace sgpp_hip
