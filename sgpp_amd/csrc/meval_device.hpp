@@ -190,20 +190,26 @@ class DeviceMultiEval {
     void* recs = nullptr;    size_t recs_cap = 0;
     void* chunks = nullptr;  size_t chunks_cap = 0;
     void* groups = nullptr;  size_t groups_cap = 0;
-    int nchunks = 0, ngroups = 0;
-    int lds = 0;        // bytes of the largest chunk's tables
-    bool wide = false;  // several data points per lane
+    void* items = nullptr;   size_t items_cap = 0;  // multTranspose: blocks, final sums
+    void* sums = nullptr;    size_t sums_cap = 0;
+    size_t part = 0;  // bytes of the items' partial sums
+    int nitems = 0, nsums = 0, segs = 0;
+    int ngroups = 0;
+    int lds = 0;  // bytes of the largest chunk's tables
   };
-  bool set_tree(const TreeGrid& g, bool multT);
+  bool set_tree(const TreeGrid& g, bool mult, bool multT);
   // Kernels that evaluate a direction: the algorithm's own or the
   // subspace tree's
   enum class Path { Own, Tree };
   bool set_paths(const TreeGrid* tree, const std::vector<double>& li,
                  const std::vector<uint32_t>& pmask);
-  bool tree_pays(const TreeGrid& g, const std::vector<double>& li,
-                 const std::vector<uint32_t>& pmask) const;
+  double culled_cost(const std::vector<double>& li, const std::vector<uint32_t>& pmask) const;
   template <typename T>
-  void set_tree_plans(const TreeGrid& g, bool multT);
+  void set_tree_plans(const TreeGrid& g, bool mult, bool multT);
+  template <typename T>
+  void set_tree_mult(const TreeGrid& g, int64_t rb, int64_t slots);
+  template <typename T>
+  void set_tree_multT(const TreeGrid& g, int64_t batches);
   void upload_tree(const TreeProgram& p, TreePlan& plan, int entry_bytes);
   template <typename T>
   void run_tree_mult(const double* d_alpha, double* d_result, hipEvent_t* tev,
@@ -271,6 +277,12 @@ class DeviceMultiEval {
   int tree_depth_ = 0;
   void* tree_ti_ = nullptr;  size_t tree_ti_cap_ = 0;
   TreePlan tree_mult_[2], tree_multT_[2];
+  // per precision the data as the walks read them (tree_points_kernel), the
+  // caller's row of each row, the number of rows
+  void* tree_x_[2] = {nullptr, nullptr};      size_t tree_x_cap_[2] = {0, 0};
+  void* tree_sperm_[2] = {nullptr, nullptr};  size_t tree_sperm_cap_[2] = {0, 0};
+  int64_t tree_rows_[2] = {0, 0};
+  bool tree_wide_[2] = {false, false};  // several data points per lane
   // boxes of a few data groups ([n][D][2]), to estimate what culling leaves
   std::vector<double> probe_boxes_;
 

@@ -54,7 +54,7 @@ namespace sgpp_hip {
 
 namespace {
 // data groups whose boxes estimate what culling leaves
-constexpr size_t kProbeGroups = 16;
+constexpr size_t kProbeGroups = 64;
 }  // namespace
 
 // Morton order of n points in [0,1]^d (row-major): b = min(16, 64/d) bits
@@ -291,11 +291,11 @@ DeviceMultiEval::~DeviceMultiEval() {
   void* bufs[] = {X64_,   X32_,   WB64_,  WB32_,  LI64_,    LI32_,   TB64_,
                   TB32_,  scale_, perm_,  pm_,    dperm_,   A_,      Y_,
                   part_,  hin_,   hout_,  sub_desc_, sub_ti_, sub_te_, sub_tw_,
-                  sub_chunk_, tree_ti_};
+                  sub_chunk_, tree_ti_, tree_x_[0], tree_x_[1], tree_sperm_[0], tree_sperm_[1]};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (TreePlan* p : {&tree_mult_[0], &tree_mult_[1], &tree_multT_[0], &tree_multT_[1]})
-    for (void* b : {p->recs, p->chunks, p->groups})
+    for (void* b : {p->recs, p->chunks, p->groups, p->items, p->sums})
       if (b) (void)hipFree(b);
   for (auto* pool : {&tm_mult_, &tm_multT_})
     for (auto& e : *pool) {
@@ -411,36 +411,69 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   }
 }
 
-// The walk of the subspace tree costs about kTreeCost operations per node and
-// data point whatever the data; the culled kernels two per evaluated dimension
-// and 2.5 more per grid point that a data group's box meets, estimated on a few
-// groups and grid points: on a d=8 grid of level 6 67 per node (FP32 mult 1,028
-// to 278 us), on an adaptive d=10 one 7 in FP64 (start 378 us, 280 us walked).
-constexpr double kTreeCost = 8.0;
-constexpr size_t kProbePoints = 16384;
-// multTranspose of the tree adds to LDS per node: it gains over the culled
-// kernel where launches count (1.3e6 nodes times data points, d=5, both products:
-// 329 to 60 us), not on a d=8 grid of level 6 (1,297 to 1,653 us).
-constexpr double kTreeMultTWork = 1e7;
+// The subspace tree's walks cost the same per node and data point whatever the
+// data; the culled kernels' cost follows the grid points that a data group's box
+// meets, estimated on a few groups and grid points (two per evaluated dimension and
+// 2.5 more, per node). Culled against walked, mult and multTranspose in us:
+//   cost   7, d=10, 1,880 nodes, M=5e6, FP32   2,295 to 3,184   2,447 to 4,671
+//   cost  11, d=10, 3,418 nodes, M=5e6, FP32   7,185 to 6,049   7,493 to 8,730
+//   cost  15, d=10, 3,418 nodes, M=1e6, FP32   2,051 to 1,403   2,218 to 1,880
+//   cost  16, d=20, 14,650 nodes, M=5e6, FP32 38,185 to 29,890  30,118 to 47,319
+//   cost  24, d=20, 14,650 nodes, M=5e5, FP32  6,523 to 3,023   5,326 to 4,917
+//   cost   6, d=10, 9,212 nodes up to 7 dimensions refined, M=2e6, FP32
+//                                              3,355 to 14,501  3,623 to 20,853
+//   cost  12, the same with 1,223 nodes, d=8, FP64
+//                                              4,055 to 2,105   4,162 to 3,184
+//   cost 109, d=8, 1,287 nodes, M=5e5, FP32    1,179 to 246     1,621 to 469
+// Below kTreeSmallWork nodes times data points the culled kernels are bound by
+// their tests and launches and the walks won at every cost measured (8 and more).
+constexpr double kTreeSmallWork = 2e9;
+constexpr double kTreeCostSmall = 5.0;
+// the cost above which a walk is the faster ({mult, multTranspose}; walks of more
+// than kTreeFewDims refined dimensions take one data point per lane)
+struct TreeCosts {
+  double mult, multT;
+};
+TreeCosts tree_costs(bool fp32, bool wide_dims, bool deep) {
+  if (fp32) return deep ? TreeCosts{22.0, 30.0} : TreeCosts{11.0, wide_dims ? 22.0 : 13.5};
+  return deep ? TreeCosts{9.0, 12.0} : TreeCosts{7.0, 10.0};
+}
+constexpr size_t kProbePoints = 2048;
+// A table larger than a block's LDS is walked in parts; beyond this many walks
+// per node the subspace algorithm keeps its own kernels.
+constexpr int64_t kTreePartWalks = 4;
 
 // Chooses the kernels of each direction (Path) and lays the grid out for them;
 // false if a direction is left to those of the instance's algorithm.
 bool DeviceMultiEval::set_paths(const TreeGrid* tree, const std::vector<double>& li,
                                 const std::vector<uint32_t>& pmask) {
   mult_path_ = multT_path_ = Path::Own;
-  const double work = tree ? static_cast<double>(tree->node.size()) * static_cast<double>(M_) : 0.0;
-  const bool small = D_ > static_cast<size_t>(kMaxTemplD) || work <= kTreeMultTWork;
-  if (tree && (algorithm_ == Algorithm::Subspace || tree_pays(*tree, li, pmask)) &&
-      set_tree(*tree, small)) {
-    mult_path_ = Path::Tree;
-    if (small) multT_path_ = Path::Tree;
+  if (!tree) return false;
+  const int64_t nodes = static_cast<int64_t>(tree->node.size());
+  const int64_t wm = tree_walks(*tree, false), wt = tree_walks(*tree, true);
+  bool mult = true, multT = true;
+  if (algorithm_ == Algorithm::Subspace) {
+    mult = wm <= kTreePartWalks * nodes;
+    multT = wt <= kTreePartWalks * nodes;
+  } else if (D_ <= static_cast<size_t>(kMaxTemplD)) {
+    const double cost = culled_cost(li, pmask);
+    const bool large = static_cast<double>(nodes) * static_cast<double>(M_) > kTreeSmallWork;
+    const TreeCosts t = large ? tree_costs(serves(Precision::FP32), D_ > 10,
+                                           tree->depth > kTreeFewDims)
+                              : TreeCosts{kTreeCostSmall, kTreeCostSmall};
+    mult = cost > t.mult * static_cast<double>(wm);
+    multT = cost > t.multT * static_cast<double>(wt);
+  }
+  if ((mult || multT) && set_tree(*tree, mult, multT)) {
+    if (mult) mult_path_ = Path::Tree;
+    if (multT) multT_path_ = Path::Tree;
   }
   return mult_path_ != Path::Own && multT_path_ != Path::Own;
 }
 
-bool DeviceMultiEval::tree_pays(const TreeGrid& g, const std::vector<double>& li,
-                                const std::vector<uint32_t>& pmask) const {
-  if (D_ > static_cast<size_t>(kMaxTemplD)) return true;
+// the estimated cost of the culled kernels per data point
+double DeviceMultiEval::culled_cost(const std::vector<double>& li,
+                                    const std::vector<uint32_t>& pmask) const {
   const size_t N = pmask.size(), step = (N + kProbePoints - 1) / kProbePoints;
   const size_t n = probe_boxes_.size() / (D_ * 2);
   double cost = 0.0;
@@ -455,8 +488,7 @@ bool DeviceMultiEval::tree_pays(const TreeGrid& g, const std::vector<double>& li
       if (hit) cost += 2.0 * __builtin_popcount(pmask[j]) + 2.5;
     }
   }
-  cost *= static_cast<double>(step) / static_cast<double>(n);
-  return kTreeCost * static_cast<double>(g.node.size()) < cost;
+  return cost * static_cast<double>(step) / static_cast<double>(n);
 }
 
 // Block order of the templated mult and multTranspose kernels (the same

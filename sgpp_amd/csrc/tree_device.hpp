@@ -31,14 +31,19 @@ namespace sgpp_hip {
 // Levels above 1 of one level vector at most (the register sets of a walk);
 // deeper grids are left to the other kernels.
 constexpr int kTreeMaxDepth = 12;
+// of the usual walks
+constexpr int kTreeFewDims = 6;
 
 // threads of a mult block (four waves share one chunk's tables)
 constexpr int kTreeBlock = 256;
 
+// multTranspose joins the values of 2^kTreeJoin lanes
+constexpr int kTreeJoin = 1;
+
 // ctl of a record
 constexpr uint32_t kTreeShiftMask = 31u;    // 33 - level
 constexpr int kTreeDimShift = 8;            // 6 bits: the dimension
-constexpr uint32_t kTreeRun = 1u << 16;     // first of its (parent, dimension): fetch x, the parent's product
+constexpr uint32_t kTreeRun = 1u << 16;     // first of its (parent, dimension): fetch its values
 constexpr uint32_t kTreeTable = 1u << 17;   // the subspace has grid points (absent parents are walked without)
 constexpr uint32_t kTreePush = 1u << 18;    // children follow
 constexpr uint32_t kTreeLast = 1u << 19;    // last of its parent's children
@@ -49,8 +54,8 @@ constexpr uint32_t kTreePart = 1u << 21;    // (without kTreeTable) part of a ta
 struct alignas(16) TreeRec {
   uint32_t off;    // byte offset of the subspace's table in the chunk's LDS image
   uint32_t ctl;
-  uint32_t scale;  // 2^(level - 1): the float's bits, or the double's upper word
-  uint32_t from;   // a run's first record: the dimensions [from, dim) to pass (Linear)
+  uint32_t scale;  // 2^(level - 1) / 2^32: the float's bits, or the double's upper word
+  uint32_t pad;
 };
 static_assert(sizeof(TreeRec) == 16, "one record is 16 bytes");
 
@@ -66,6 +71,22 @@ struct alignas(16) TreeChunk {
   int root, part;
 };
 static_assert(sizeof(TreeChunk) == 32, "one chunk is 32 bytes");
+
+// A multTranspose block: batches [b0, b1) of 64 * K rows for one chunk, whose
+// sums go to part[off, off + n).
+struct alignas(16) TreeItem {
+  int chunk, b0, b1, pad;
+  long long off, pad2;
+};
+static_assert(sizeof(TreeItem) == 32, "one item is 32 bytes");
+
+// The partial sums of up to 64 table entries of a chunk: rows of stride ld, the
+// first at off; entries [e0, e0 + n) of the tables.
+struct alignas(16) TreeSum {
+  int n, rows;
+  long long off, ld, e0;
+};
+static_assert(sizeof(TreeSum) == 32, "one sum is 32 bytes");
 
 // A grid's subspaces in walking order, and their tables.
 struct TreeGrid {
@@ -89,6 +110,10 @@ struct TreeGrid {
 bool build_tree_grid(size_t D, size_t N, const uint32_t* level, const uint32_t* index,
                      bool quiet, TreeGrid& g);
 
+// Nodes to walk per data point, those of tables in parts counted per part (and
+// their ancestors).
+int64_t tree_walks(const TreeGrid& g, bool multT);
+
 // Programs of a grid: groups of chunks of at most cap table entries and
 // max_nodes nodes; the groups have about equal numbers of nodes.
 struct TreeProgram {
@@ -101,8 +126,8 @@ TreeProgram build_tree_program(const TreeGrid& g, int ngroups, int64_t cap, int6
                                int entry_bytes, bool fp32);
 
 struct TreeMultArgs {
-  const void* X;  // [D][ldx], stored order
-  int64_t ldx, M;
+  const void* X;  // [rows of ldx]: tree_points_kernel
+  int64_t ldx;
   int D;
   const TreeRec* recs;
   const TreeChunk* chunks;
@@ -111,9 +136,9 @@ struct TreeMultArgs {
   const void* W;      // weights in table order and compute type, or null:
   const double* alpha;  // gathered from here through ti
   const int32_t* ti;
-  double* part;  // [gridDim.y][ldx], or null: results to out[dperm[m]]
+  double* part;  // [gridDim.y][ldx], or null: results to out[sperm[row]]
   double* out;
-  const int32_t* dperm;
+  const int32_t* sperm;  // the caller's row, -1 for padding
   int zero_off;  // byte offset of an LDS zero (rows outside a part)
 };
 
@@ -121,12 +146,11 @@ struct TreeMultTArgs {
   const void* X;
   int64_t ldx;
   int D;
-  const void* Y;  // [ldx] stored order, compute type, 0 past the data
+  const void* Y;  // [ldx] in X's order and type, 0 in padding rows
   const TreeRec* recs;
   const TreeChunk* chunks;
-  int64_t seg, mend;  // rows per segment (blockIdx.y), end of the rows
-  double* part;       // [segments][ntable]
-  int64_t ntable;
+  const TreeItem* items;  // one per block
+  double* part;
 };
 
 // Launchers of one compute type and basis. wide: several data points per
@@ -135,8 +159,7 @@ struct TreeMultTArgs {
 struct TreeLaunch {
   int k = 1;
   void (*mult)(const TreeMultArgs&, dim3 grid, unsigned block, unsigned lds, hipStream_t s) = nullptr;
-  int kt = 1;
-  void (*multT)(const TreeMultTArgs&, dim3 grid, unsigned lds, hipStream_t s) = nullptr;
+  void (*multT)(const TreeMultTArgs&, unsigned items, unsigned lds, hipStream_t s) = nullptr;
 };
 template <typename T, bool kMod>
 TreeLaunch tree_launch(int D, int depth, bool wide);

@@ -17,29 +17,18 @@ namespace {
 typedef unsigned TreeRecWords __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(4))) TreeRecWords* TreeRecPtr;
 
-// one instruction each: the C++ forms add a range check or a canonicalisation
-__device__ __forceinline__ unsigned to_fixed(float x) {  // floor(x 2^32), 2^32 - 1 at x = 1
+// one instruction: the C++ form adds a range check (2^32 gives 2^32 - 1)
+__device__ __forceinline__ unsigned to_fixed(float x) {
   unsigned r;
-  const float s = x * 4294967296.0f;
-  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(s));
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
   return r;
 }
 __device__ __forceinline__ unsigned to_fixed(double x) {
   unsigned r;
-  const double s = x * 4294967296.0;
-  asm("v_cvt_u32_f64 %0, %1" : "=v"(r) : "v"(s));
+  asm("v_cvt_u32_f64 %0, %1" : "=v"(r) : "v"(x));
   return r;
 }
-__device__ __forceinline__ float max_raw(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ double max_raw(double a, double b) {
-  double r;
-  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
+// one instruction each (no canonicalisation): min(a, b), max(|a|, b)
 __device__ __forceinline__ float min_raw(float a, float b) {
   float r;
   asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
@@ -50,17 +39,21 @@ __device__ __forceinline__ double min_raw(double a, double b) {
   asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
   return r;
 }
+__device__ __forceinline__ float max_abs(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, |%1|, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double max_abs(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, |%1|, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 __device__ __forceinline__ float rint_raw(float a) { return __builtin_rintf(a); }
 __device__ __forceinline__ double rint_raw(double a) { return __builtin_rint(a); }
 __device__ __forceinline__ float scale_of(uint32_t bits, float) { return __uint_as_float(bits); }
 __device__ __forceinline__ double scale_of(uint32_t bits, double) {
   return __hiloint2double(static_cast<int>(bits), 0);
-}
-
-// the level-1 hat at x
-template <typename T>
-__device__ __forceinline__ T level_one(T x) {
-  return min_raw(x + x, T(2) - (x + x));
 }
 
 // Values indexed by a wave-uniform dimension, in registers: 32-bit words in
@@ -117,83 +110,81 @@ __device__ __forceinline__ void dim_values(const DimRegs<T, DB> (&v)[K], int r, 
   dim_values<T, DB, K, 1>(vs, r, outs);
 }
 
-// The data points of a walk: coordinates in registers (DB > 0), and for
-// Linear grids the products rest[d] of the level-1 factors of the dimensions
-// after d; or (DB == 0, many dimensions) read from memory when a run begins.
-// one[k]: the product of all level-1 factors (1 for ModLinear).
+// The data points of a walk, as tree_points_kernel stores them: per dimension
+// the coordinate times 2^32 and, for Linear grids, 2 over the level-1 factor, in
+// registers (DB > 0) or, for many dimensions (DB == 0), read from memory when a
+// run begins; and the product of all level-1 factors.
 template <typename T, int DB, int K, bool kMod>
 struct TreePoints {
-  DimRegs<T, DB> x[K];
-  DimRegs<T, DB> rest[kMod ? 1 : K];
+  DimRegs<T, DB> x[K], c[kMod ? 1 : K];
   __device__ __forceinline__ void load(const T* __restrict__ X, int64_t ldx, int D, int64_t m,
                                        T (&one)[K]) {
-    T v[K][DB];
 #pragma unroll
-    for (int d = 0; d < DB; ++d)
+    for (int k = 0; k < K; ++k) one[k] = kMod ? T(1) : X[2 * D * ldx + m + k * 64];
 #pragma unroll
-      for (int k = 0; k < K; ++k) v[k][d] = d < D ? X[d * ldx + m + k * 64] : T(0.5);
+    for (int d = 0; d < DB; ++d) {
+      const int from = min(d, D - 1);  // (the rest are not read; no branches)
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      one[k] = T(1);
-#pragma unroll
-      for (int d = DB - 1; d >= 0; --d) {
-        x[k].set(d, v[k][d]);
-        if constexpr (!kMod) {
-          rest[k].set(d, one[k]);
-          one[k] *= level_one(v[k][d]);  // (1 at the unused dimensions' 1/2)
-        }
+      for (int k = 0; k < K; ++k) {
+        x[k].set(d, X[from * ldx + m + k * 64]);
+        if constexpr (!kMod) c[k].set(d, X[(D + from) * ldx + m + k * 64]);
       }
     }
   }
-  __device__ __forceinline__ void coordinates(int r, T (&xr)[K]) const {
-    dim_values(x, r, xr);
+  __device__ __forceinline__ void values(int r, T (&xr)[K], T (&cr)[K]) const {
+    if constexpr (kMod) {
+      const DimRegs<T, DB>(*const v[1])[K] = {&x};
+      T(*const out[1])[K] = {&xr};
+      dim_values<T, DB, K, 1>(v, r, out);
+    } else {
+      const DimRegs<T, DB>(*const v[2])[K] = {&x, &c};
+      T(*const out[2])[K] = {&xr, &cr};
+      dim_values<T, DB, K, 2>(v, r, out);
+    }
   }
-  // the level-1 factors after dimension r
-  __device__ __forceinline__ void after(int r, int, T (&s)[K]) const { dim_values(rest, r, s); }
 };
 template <typename T, int K, bool kMod>
 struct TreePoints<T, 0, K, kMod> {
   const T* p;
   int64_t ld;
+  int dims;
   __device__ __forceinline__ void load(const T* __restrict__ X, int64_t ldx, int D, int64_t m,
                                        T (&one)[K]) {
     p = X + m;
     ld = ldx;
+    dims = D;
 #pragma unroll
-    for (int k = 0; k < K; ++k) one[k] = T(1);
-    if constexpr (!kMod) after(-1, D, one);
+    for (int k = 0; k < K; ++k) one[k] = kMod ? T(1) : p[2 * D * ldx + k * 64];
   }
-  __device__ __forceinline__ void coordinates(int r, T (&xr)[K]) const {
+  __device__ __forceinline__ void values(int r, T (&xr)[K], T (&cr)[K]) const {
 #pragma unroll
-    for (int k = 0; k < K; ++k) xr[k] = p[r * ld + k * 64];
-  }
-  __device__ __forceinline__ void after(int r, int D, T (&s)[K]) const {
-#pragma unroll
-    for (int k = 0; k < K; ++k) s[k] = T(1);
-    for (int d = D - 1; d > r; --d)
-#pragma unroll
-      for (int k = 0; k < K; ++k) s[k] *= level_one(p[d * ld + k * 64]);
+    for (int k = 0; k < K; ++k) {
+      xr[k] = p[r * ld + k * 64];
+      if constexpr (!kMod) cr[k] = p[(dims + r) * ld + k * 64];
+    }
   }
 };
 
-// The walk over a chunk's program. Per depth the parent's product R (of the
-// factors of the dimensions up to its last step; for Linear grids extended by
-// the level-1 factors of the dimensions passed since) and table position F. A
-// run (the children of one parent in one dimension) fetches x, its 32-bit
-// fixed-point form (the cell of level l is its top l - 1 bits) and rr, the
-// product of all factors but the run's own. Per node and data point:
-//   t = 2^(l-1) x - 1/2, w = t - rint(t) in [-1/2, 1/2]: the hat is 1 - 2|w|
-//   ModLinear: its extrapolated boundary functions are 2 - 2^l min(x, 1-x),
-//   which exceeds the hat in the boundary cells only: the larger of the two.
+// The walk over a chunk's program. Per depth the product R of all factors of
+// the subspace at that depth (level 1 in the dimensions not refined) and its
+// table position F. A run (the children of one parent in one dimension)
+// fetches x 2^32, whose integer part's top l - 1 bits are the cell of level l,
+// and rr, twice the product of all factors but the run's own. Per node and
+// data point, with v = 2^(l-1) x (its cells are the unit intervals):
+//   Linear: half the hat is |v - rint(v)|, the distance to the nearest cell
+//     edge (exact); R times 2 over the dimension's level-1 factor takes that
+//     factor out.
+//   ModLinear: level-1 factors are 1. The extrapolated boundary functions are
+//     2 - 2^l min(x, 1-x), which exceeds the hat in the boundary cells only:
+//     the larger of the two.
 // A point on a cell edge may round to either side: the hat is 0 there.
 template <typename T, int DB, int K, bool kMod, int MD, typename Use>
 struct TreeWalk {
   TreePoints<T, DB, K, kMod>& pts;
-  Use& use;
+  Use use;
   TreeRecPtr next;
   TreeRecWords cur;
-  int D;
-  T xr[K], rr[K], xm[K];
+  T xr[K], cr[K], rr[K];
   unsigned fx[K];
 
   __device__ __forceinline__ void run(TreeRecPtr recs, const T (&R0)[K]) {
@@ -206,30 +197,18 @@ struct TreeWalk {
   }
 
   template <int kDepth>
-  __device__ __forceinline__ void level(const T (&R0)[K], const unsigned (&F)[K]) {
-    T R[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) R[k] = R0[k];
+  __device__ __forceinline__ void level(const T (&R)[K], const unsigned (&F)[K]) {
     for (;;) {
-      const unsigned off = cur.x, ctl = cur.y, scale = cur.z, from = cur.w;
+      const unsigned off = cur.x, ctl = cur.y, scale = cur.z;
       ++next;
       cur = next[0];  // in flight during this node
       if (ctl & kTreeRun) {
-        const int r = (ctl >> kTreeDimShift) & 63u;
-        if constexpr (!kMod) {
-          for (int d = static_cast<int>(from); d < r; ++d) {
-            pts.coordinates(d, xr);
-#pragma unroll
-            for (int k = 0; k < K; ++k) R[k] *= level_one(xr[k]);
-          }
-          pts.after(r, D, rr);
-        }
-        pts.coordinates(r, xr);
+        pts.values((ctl >> kTreeDimShift) & 63u, xr, cr);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           fx[k] = to_fixed(xr[k]);
-          rr[k] = kMod ? R[k] : R[k] * rr[k];
-          if constexpr (kMod) xm[k] = level_one(xr[k]);
+          if constexpr (kMod) cr[k] = min_raw(xr[k], T(4294967296.0) - xr[k]);
+          rr[k] = kMod ? R[k] + R[k] : R[k] * cr[k];
         }
       }
       unsigned E[K];
@@ -237,25 +216,18 @@ struct TreeWalk {
       for (int k = 0; k < K; ++k) E[k] = __builtin_amdgcn_alignbit(F[k], fx[k], ctl);
       use.begin(off, ctl, E);
       const T L = scale_of(scale, T(0));
-      T f[K], P[K];
+      T P[K];
 #pragma unroll
       for (int k = 0; k < K; ++k) {
-        const T t = fmaT(xr[k], L, T(-0.5));
-        const T w = t - rint_raw(t);
-        f[k] = fmaT(T(-2), absT(w), T(1));
-        if constexpr (kMod) f[k] = max_raw(f[k], fmaT(-L, xm[k], T(2)));
-        P[k] = rr[k] * f[k];
+        const T v = xr[k] * L;
+        const T e = v - rint_raw(v);
+        P[k] = rr[k] * (kMod ? max_abs(e, fmaT(-L, cr[k], T(1))) : absT(e));
       }
       use.end(off, ctl, P, E);
       if (ctl & (kTreePush | kTreeLast | kTreeFlush)) {
         if (sizeof(T) == 4 && (ctl & kTreeFlush)) use.flush();
         if constexpr (kDepth + 1 < MD)
-          if (ctl & kTreePush) {
-            if constexpr (!kMod)
-#pragma unroll
-              for (int k = 0; k < K; ++k) P[k] = R[k] * f[k];
-            level<kDepth + 1>(P, E);
-          }
+          if (ctl & kTreePush) level<kDepth + 1>(P, E);
         if (ctl & kTreeLast) return;
       }
     }
@@ -304,14 +276,15 @@ struct TreeGather {
   }
 };
 
-// mult: bound by vector instructions, ten to fourteen per node and data point
-// (one scalar instruction issues in four cycles, so several points per lane
-// share a node's); the weights of a chunk's subspaces are gathered from LDS,
-// where up to 64 cells meet no bank conflict. Against evaluating every
-// dimension of each grid point that a wave's box meets (kernel times): FP32,
-// Linear d=8 level 6, 5e5 data points 1,028 to 260 us; FP64, the same 1,452 to
-// 440 us, ModLinear d=7 level 6, 2.5e5 points 360 to 147 us, Linear d=30 level
-// 3, 5e4 points 1,262 to 131 us.
+// mult: bound by vector instructions, most of which issue every four cycles in
+// either precision: seven (Linear) or nine per node and data point and four per run
+// (one scalar instruction issues in four cycles, so several points per lane share
+// a node's). The weights of a chunk's subspaces are gathered from LDS, where up to
+// 64 cells meet no bank conflict. Kernel times against the culled kernels: Linear
+// d=8 level 6, 5e5 points, FP32 1,179 to 246 us, FP64 1,678 to 378; d=20 adaptive,
+// 5e5 points, FP32 6,523 to 3,023; ModLinear d=10 adaptive, 1e6 points, FP32 2,051
+// to 1,403. Factors relative to the level-1 ones, instead of extending each product
+// by the dimensions passed: d=20 4,960 to 3,020, d=8 284 to 246 us.
 template <typename T, int DB, int K, bool kMod, int MD>
 __global__ __launch_bounds__(kTreeBlock) __attribute__((amdgpu_waves_per_eu(kMod ? 4 : 3)))
 void tree_mult_kernel(const TreeMultArgs a) {
@@ -320,14 +293,13 @@ void tree_mult_kernel(const TreeMultArgs a) {
   const int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x * K + wave * 64 * K + lane;
   T* lds = reinterpret_cast<T*>(tree_lds);
   TreePoints<T, DB, K, kMod> pts;
-  T all[K], one[K];
+  T all[K];
   pts.load(static_cast<const T*>(a.X), a.ldx, a.D, m, all);
   TreeGather<T, K> g;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     g.acc[k] = T(0);
     g.accd[k] = 0.0;
-    one[k] = T(1);
   }
   g.zero_off = a.zero_off;
   const int g0 = blockIdx.y * a.gper;
@@ -352,11 +324,12 @@ void tree_mult_kernel(const TreeMultArgs a) {
     if (ch.root) {
       const T w = lds[0];
 #pragma unroll
-      for (int k = 0; k < K; ++k) g.accd[k] += static_cast<double>(kMod ? w : w * all[k]);
+      for (int k = 0; k < K; ++k) g.accd[k] += static_cast<double>(w * all[k]);
     }
     if (ch.nrec > 0) {
-      TreeWalk<T, DB, K, kMod, MD, TreeGather<T, K>> walk{pts, g, nullptr, TreeRecWords{}, a.D};
-      walk.run((TreeRecPtr)(a.recs + ch.rec0), one);
+      TreeWalk<T, DB, K, kMod, MD, TreeGather<T, K>> walk{pts, g, nullptr, TreeRecWords{}};
+      walk.run((TreeRecPtr)(a.recs + ch.rec0), all);
+      g = walk.use;
       g.flush();
     }
   }
@@ -366,109 +339,108 @@ void tree_mult_kernel(const TreeMultArgs a) {
     const int64_t row = m + k * 64;
     if (a.part)
       a.part[static_cast<int64_t>(blockIdx.y) * a.ldx + row] = r;
-    else if (row < a.M)
-      a.out[a.dperm[row]] = r;
+    else if (const int32_t j = a.sperm[row]; j >= 0)
+      a.out[j] = r;
   }
 }
 
-// multTranspose: the sums over the wave's data points of each table position
-// they fall in. Morton order puts most waves into one or two positions of a
-// subspace: per position, the lanes' points are added, summed over the lanes
-// (DPP) and added to the wave's own tables in LDS, in FP64 and in a fixed
-// order (repeats are bit-identical).
+// v with all bits kept or cleared
+__device__ __forceinline__ float and_bits(float v, unsigned m) {
+  return __uint_as_float(__float_as_uint(v) & m);
+}
+__device__ __forceinline__ double and_bits(double v, unsigned m) {
+  return __hiloint2double(static_cast<int>(static_cast<unsigned>(__double2hiint(v)) & m),
+                          static_cast<int>(static_cast<unsigned>(__double2loint(v)) & m));
+}
+
+// multTranspose: each data point's value is added to its table position, in
+// LDS, in FP64. Equal positions in one LDS add wait for each other (64 equal
+// ones 192 cycles, 64 different ones 9), so values are joined first: the points
+// of a pair of lanes are consecutive in storage order (tree_points_kernel) and
+// mostly in one position; the pairs are far apart. Joining two or three steps more
+// cost more instructions than the conflicts they saved (d=8 level 6, FP64:
+// 706 and 767 us against 675), none at all cost 667 against 598 later.
 template <typename T, int K>
 struct TreeScatter {
   unsigned part0, partn;
-  int lane;
+  unsigned keep;  // all ones in the lane of a pair that keeps the joined value
   __device__ __forceinline__ void begin(uint32_t, uint32_t, const unsigned (&)[K]) {}
   __device__ __forceinline__ void flush() {}
   __device__ __forceinline__ void add(unsigned byte, T c) {
-    const T s = sum_to_lane63(c);
-    if (lane == 63)
-      atomicAdd(reinterpret_cast<double*>(tree_lds + byte), static_cast<double>(s));
+    atomicAdd(reinterpret_cast<double*>(tree_lds + byte), static_cast<double>(c));
   }
   __device__ __forceinline__ void end(uint32_t off, uint32_t ctl, const T (&P)[K],
                                       const unsigned (&E)[K]) {
-    unsigned long long rem[K];
-    if (!(ctl & kTreeTable)) {
-      if (!(ctl & kTreePart)) return;
+    if (ctl & kTreeTable) {
+      T v[K];
 #pragma unroll
-      for (int k = 0; k < K; ++k) rem[k] = __ballot(E[k] - part0 < partn);
-    } else {
-      const unsigned e0 =
-          static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(E[0])));
-      unsigned long long other = 0ull;
+      for (int k = 0; k < K; ++k) v[k] = P[k];
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        rem[k] = ~0ull;
-        other |= __ballot(E[k] != e0);
-      }
-      if (other == 0ull) {
-        T c = P[0];
+      for (int w = 1; w < K; w *= 2)
 #pragma unroll
-        for (int k = 1; k < K; ++k) c += P[k];
-        add(off + e0 * 8u, c);
-        return;
-      }
-    }
-    for (;;) {
-      unsigned e0 = 0u;
-      bool any = false;
+        for (int k = 0; k + w < K; k += 2 * w) {
+          const bool differ = E[k] != E[k + w];
+          T c = differ ? T(0) : v[k + w];
+          asm("" : "+v"(c));  // (a select, not a branch)
+          if (__ballot(differ) != 0ull)
+            if (differ) add(off + E[k + w] * 8u, v[k + w]);
+          v[k] += c;
+        }
+      static_assert(kTreeJoin == 1, "lanes join in pairs");
+      constexpr int kPair = 0xb1;  // quad_perm [1,0,3,2]
+      const unsigned e = static_cast<unsigned>(
+          __builtin_amdgcn_mov_dpp(static_cast<int>(E[0]), kPair, 0xf, 0xf, true));
+      const T sum = and_bits(v[0] + dpp_z<kPair>(v[0]), keep);
+      v[0] = E[0] == e ? sum : v[0];
+      if (v[0] != T(0)) add(off + E[0] * 8u, v[0]);
+    } else if (ctl & kTreePart) {
 #pragma unroll
       for (int k = 0; k < K; ++k)
-        if (!any && rem[k] != 0ull) {
-          any = true;
-          e0 = static_cast<unsigned>(__builtin_amdgcn_readlane(
-              static_cast<int>(E[k]), __builtin_ctzll(rem[k])));
-        }
-      if (!any) break;
-      T c = T(0);
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const bool in = E[k] == e0;
-        rem[k] &= ~__ballot(in);
-        c += in ? P[k] : T(0);
-      }
-      add(off + e0 * 8u, c);
+        if (E[k] - part0 < partn) add(off + E[k] * 8u, P[k]);
     }
   }
 };
 
-// FP64 kernel times: d=5 level 5, 1e4 points 15 us; d=30 level 3, 5e4 points
-// 2,104 to 157 us; bound by the sums over the lanes and the LDS adds.
+// Bound by vector instructions, the LDS adds about half of the time beside them.
+// Kernel times against the culled kernel: Linear d=8 level 6, 5e5 points, FP32
+// 1,621 to 469 us, FP64 2,300 to 574; ModLinear d=10 adaptive, 1e6 points, FP32
+// 2,218 to 1,903; against the subspace algorithm's own, d=7 level 6, 2.5e5 points,
+// 681 to 224 with the final sums.
 template <typename T, int DB, int K, bool kMod, int MD>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kMod ? 4 : 3)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 void tree_multT_kernel(const TreeMultTArgs a) {
   const int lane = threadIdx.x;
-  const TreeChunk ch = a.chunks[blockIdx.x];
+  const TreeItem it = a.items[blockIdx.x];
+  const TreeChunk ch = a.chunks[it.chunk];
   double* acc = reinterpret_cast<double*>(tree_lds);
   for (int i = lane; i < ch.n; i += 64) acc[i] = 0.0;
   TreeScatter<T, K> sc;
   sc.part0 = ch.part0;
   sc.partn = ch.n;
-  sc.lane = lane;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * a.seg;
-  const int64_t m1 = m0 + a.seg < a.mend ? m0 + a.seg : a.mend;
-  for (int64_t mb = m0; mb < m1; mb += 64 * K) {
-    const int64_t m = mb + lane;
+  sc.keep = lane & 1 ? 0u : ~0u;
+  for (int b = it.b0; b < it.b1; ++b) {
+    const int64_t m = static_cast<int64_t>(b) * (64 * K) + lane;
     TreePoints<T, DB, K, kMod> pts;
     T y[K], all[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) y[k] = static_cast<const T*>(a.Y)[m + k * 64];
     pts.load(static_cast<const T*>(a.X), a.ldx, a.D, m, all);
+#pragma unroll
+    for (int k = 0; k < K; ++k) y[k] *= all[k];
     if (ch.root) {
       T c = T(0);
 #pragma unroll
-      for (int k = 0; k < K; ++k) c = fmaT(y[k], all[k], c);
-      sc.add(0u, c);
+      for (int k = 0; k < K; ++k) c += y[k];
+      c = sum_to_lane63(c);
+      if (lane == 63) sc.add(0u, c);
     }
     if (ch.nrec > 0) {
-      TreeWalk<T, DB, K, kMod, MD, TreeScatter<T, K>> walk{pts, sc, nullptr, TreeRecWords{}, a.D};
+      TreeWalk<T, DB, K, kMod, MD, TreeScatter<T, K>> walk{pts, sc, nullptr, TreeRecWords{}};
       walk.run((TreeRecPtr)(a.recs + ch.rec0), y);
     }
   }
   // (one wave: its LDS operations are in order)
-  double* out = a.part + static_cast<int64_t>(blockIdx.y) * a.ntable + ch.off0;
+  double* out = a.part + it.off;
   for (int i = lane; i < ch.n; i += 64) out[i] = acc[i];
 }
 
@@ -479,9 +451,9 @@ void launch_tree_mult(const TreeMultArgs& a, dim3 grid, unsigned block, unsigned
   hipLaunchKernelGGL((tree_mult_kernel<T, DB, K, kMod, MD>), grid, dim3(block), lds, s, a);
 }
 template <typename T, int DB, int K, bool kMod, int MD>
-void launch_tree_multT(const TreeMultTArgs& a, dim3 grid, unsigned lds, hipStream_t s) {
+void launch_tree_multT(const TreeMultTArgs& a, unsigned items, unsigned lds, hipStream_t s) {
   clear_launch_error();
-  hipLaunchKernelGGL((tree_multT_kernel<T, DB, K, kMod, MD>), grid, dim3(64), lds, s, a);
+  hipLaunchKernelGGL((tree_multT_kernel<T, DB, K, kMod, MD>), dim3(items), dim3(64), lds, s, a);
 }
 
 // data points per lane of the wide variants
@@ -493,13 +465,13 @@ constexpr int tree_k(int DB) {
 template <typename T, bool kMod, int DB>
 TreeLaunch tree_variant(int depth, bool wide) {
   constexpr int K = tree_k<T>(DB == 0 ? 20 : DB);
-  constexpr int kFew = DB == 4 ? 4 : 6;  // register sets of the usual variants
+  constexpr int kFew = DB == 4 ? 4 : kTreeFewDims;  // register sets of the usual variants
   TreeLaunch l;
   if (depth > kFew) {
     l.mult = &launch_tree_mult<T, DB, 1, kMod, kTreeMaxDepth>;
     l.multT = &launch_tree_multT<T, DB, 1, kMod, kTreeMaxDepth>;
   } else if (wide) {
-    l.k = l.kt = K;
+    l.k = K;
     l.mult = &launch_tree_mult<T, DB, K, kMod, kFew>;
     l.multT = &launch_tree_multT<T, DB, K, kMod, kFew>;
   } else {

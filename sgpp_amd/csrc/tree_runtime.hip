@@ -23,6 +23,59 @@ __global__ void tree_weights_kernel(const double* __restrict__ alpha,
   if (e < n) W[e] = ti[e] >= 0 ? static_cast<T>(alpha[ti[e]]) : T(0);
 }
 
+// The data as the walks read them, in batches of 64 K rows (row 64 k + l of a
+// batch is lane l's point k): the lanes that multTranspose joins have consecutive
+// stored rows, and such groups are spread evenly over all rows. X: [D][ldx]. XT: per
+// dimension a row of 2^32 x; for Linear grids then per dimension a row of 2 over
+// the level-1 factor, and a row of the products of the level-1 factors. Rows past
+// M are copies of row M - 1 whose caller's row sperm is -1.
+template <typename T, bool kMod>
+__global__ void tree_points_kernel(const T* __restrict__ X, int64_t ldx,
+                                   const int32_t* __restrict__ dperm, int64_t M, int D, int K,
+                                   int64_t rows, T* __restrict__ XT,
+                                   int32_t* __restrict__ sperm) {
+  // (below this a Linear level-1 factor's reciprocal could overflow)
+  constexpr double kTiny = sizeof(T) == 4 ? 0x1.0p-100 : 0x1.0p-1000;
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (r >= rows) return;
+  constexpr int kGroup = 1 << kTreeJoin, kGroups = 64 / kGroup;
+  const int lane = r % 64, k = r / 64 % K;
+  const int64_t m = (lane / kGroup) * (rows / kGroups) + r / (64 * K) * (kGroup * K) +
+                    (lane % kGroup) * K + k;
+  const int64_t from = m < M ? m : M - 1;
+  sperm[r] = m < M ? dperm[m] : -1;
+  double all = 1.0;
+  for (int d = 0; d < D; ++d) {
+    const double x = static_cast<double>(X[d * ldx + from]);
+    XT[d * rows + r] = static_cast<T>(x * 0x1.0p32);
+    if (kMod) continue;
+    const double h = 2.0 * fmin(x, 1.0 - x);
+    XT[(D + d) * rows + r] = static_cast<T>(h < kTiny ? 0.0 : 2.0 / h);
+    all *= h < kTiny ? 0.0 : h;
+  }
+  if (!kMod) XT[2 * D * rows + r] = static_cast<T>(all);
+}
+
+// Y[r] = y[sperm[r]], 0 where sperm is -1
+template <typename T>
+__global__ void tree_prep_kernel(const double* __restrict__ y, const int32_t* __restrict__ sperm,
+                                 T* __restrict__ Y, int64_t n) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (r < n) Y[r] = sperm[r] >= 0 ? static_cast<T>(y[sperm[r]]) : T(0);
+}
+
+// out[ti[e]] = the sum of a table entry's partial sums, rows added in a fixed order
+__global__ __launch_bounds__(kRows* kCols) void tree_sum_kernel(
+    const double* __restrict__ part, const TreeSum* __restrict__ sums,
+    const int32_t* __restrict__ ti, double* __restrict__ out) {
+  const TreeSum q = sums[blockIdx.x];
+  const int c = threadIdx.x % kCols;
+  const double s = sum_rows(part + q.off + c, q.ld, c < q.n ? q.rows : 0);
+  if (threadIdx.x >= kCols || c >= q.n) return;
+  const int32_t j = ti[q.e0 + c];
+  if (j >= 0) out[j] = s;
+}
+
 }  // namespace
 
 bool build_tree_grid(size_t D, size_t N, const uint32_t* level, const uint32_t* index,
@@ -167,8 +220,6 @@ void append_program(const TreeGrid& g, size_t a, size_t b, int64_t off0, int ent
                        flags});
     path = steps;
   }
-  // the dimensions that the product at each depth covers
-  int covered[kTreeMaxDepth + 2] = {};
   for (size_t i = 0; i < out.size(); ++i) {
     Emit& e = out[i];
     if (i + 1 < out.size() && out[i + 1].depth == e.depth + 1) e.flags |= kTreePush;
@@ -182,11 +233,8 @@ void append_program(const TreeGrid& g, size_t a, size_t b, int64_t off0, int ent
     r.off = e.off;
     r.ctl = static_cast<uint32_t>(33 - e.level) | (static_cast<uint32_t>(e.dim) << kTreeDimShift) |
             e.flags;
-    r.from = static_cast<uint32_t>(covered[e.depth]);
-    covered[e.depth] = e.dim;
-    covered[e.depth + 1] = e.dim + 1;
-    r.scale = fp32 ? static_cast<uint32_t>(127 + e.level - 1) << 23
-                   : static_cast<uint32_t>(1023 + e.level - 1) << 20;
+    r.scale = fp32 ? static_cast<uint32_t>(127 + e.level - 33) << 23
+                   : static_cast<uint32_t>(1023 + e.level - 33) << 20;
     p.recs.push_back(r);
   }
 }
@@ -250,18 +298,23 @@ TreeProgram build_tree_program(const TreeGrid& g, int ngroups, int64_t cap, int6
 namespace {
 
 // LDS of a mult block and of a multTranspose wave: 40 KiB and 10 KiB let the
-// registers, not the LDS, bound the waves in flight (16 per CU, 12 for Linear)
+// the registers bound the waves in flight (16 per CU, 12 for Linear)
 constexpr int kMultLds = 40 << 10;
 constexpr int kMultTEntries = 1280;
 // nodes per chunk group (mult) or chunk (multTranspose) at least, so that a
 // wave's start is small against its walk
 constexpr int kMinNodes = 8;
+// multTranspose: nodes times batches of a wave, and what a batch's loads cost in
+// nodes
+// (a d=8 regular grid, M=5e5: 2 rounds; a d=10 adaptive one, M=1e6: 2 rounds 2,058
+// us with the final sums, 4 1,949, 16 1,943)
+constexpr int64_t kMultTWork = 300;
+constexpr int kBatchNodes = 5;
 constexpr int64_t kTreePartialBudget = int64_t(2048) << 20;
 
 }  // namespace
 
 void DeviceMultiEval::upload_tree(const TreeProgram& p, TreePlan& plan, int entry_bytes) {
-  plan.nchunks = static_cast<int>(p.chunks.size());
   plan.ngroups = static_cast<int>(p.groups.size()) - 1;
   plan.lds = (p.max_entries * entry_bytes + 15) / 16 * 16;
   ensure(&plan.recs, &plan.recs_cap, p.recs.size() * sizeof(TreeRec));
@@ -279,25 +332,42 @@ void DeviceMultiEval::upload_tree(const TreeProgram& p, TreePlan& plan, int entr
 }
 
 template <typename T>
-void DeviceMultiEval::set_tree_plans(const TreeGrid& g, bool multT) {
+void DeviceMultiEval::set_tree_plans(const TreeGrid& g, bool mult, bool multT) {
   const int ix = sizeof(T) == sizeof(double) ? 0 : 1;
   const bool mod = basis_ == Basis::ModLinear;
   const int64_t nodes = static_cast<int64_t>(g.node.size());
   const int64_t M = static_cast<int64_t>(M_);
-  const int waves_cu = mod ? 16 : 12;
-  const int64_t slots = static_cast<int64_t>(num_cus_) * waves_cu;
+  const int64_t slots = static_cast<int64_t>(num_cus_) * (mod ? 16 : 12);
   auto launch = [&](bool wide) {
     return mod ? tree_launch<T, true>(static_cast<int>(D_), g.depth, wide)
                : tree_launch<T, false>(static_cast<int>(D_), g.depth, wide);
   };
   // several points per lane where that leaves every wave slot a walk of kMinNodes
   TreeLaunch l = launch(true);
-  const bool wide = M * nodes >= slots * 64 * l.k * kMinNodes;
-  l = launch(wide);
-  // mult: chunk groups so that the blocks fill the device evenly
-  TreePlan& pm = tree_mult_[ix];
-  pm.wide = wide;
+  tree_wide_[ix] = M * nodes >= slots * 64 * l.k * kMinNodes;
+  l = launch(tree_wide_[ix]);
+  // the data in the walks' order
   const int64_t rb = (M + kTreeBlock * l.k - 1) / (kTreeBlock * l.k);
+  const int64_t rows = tree_rows_[ix] = rb * kTreeBlock * l.k;
+  ensure(&tree_x_[ix], &tree_x_cap_[ix], (mod ? D_ : 2 * D_ + 1) * rows * sizeof(T));
+  ensure(&tree_sperm_[ix], &tree_sperm_cap_[ix], rows * sizeof(int32_t));
+  clear_launch_error();
+  hipLaunchKernelGGL((mod ? tree_points_kernel<T, true> : tree_points_kernel<T, false>),
+                     dim3(blocks(rows, 256)), dim3(256), 0, stream_,
+                     static_cast<const T*>(sizeof(T) == sizeof(double) ? X64_ : X32_),
+                     static_cast<int64_t>(Mpad_), static_cast<const int32_t*>(dperm_), M,
+                     static_cast<int>(D_), l.k, rows, static_cast<T*>(tree_x_[ix]),
+                     static_cast<int32_t*>(tree_sperm_[ix]));
+  check_hip(hipGetLastError(), "tree data order");
+  if (mult) set_tree_mult<T>(g, rb, slots);
+  if (multT) set_tree_multT<T>(g, rows / (64 * l.k));
+}
+
+// mult: chunk groups so that the blocks (rb per group) fill the slots evenly
+template <typename T>
+void DeviceMultiEval::set_tree_mult(const TreeGrid& g, int64_t rb, int64_t slots) {
+  TreePlan& pm = tree_mult_[sizeof(T) == sizeof(double) ? 0 : 1];
+  const int64_t nodes = static_cast<int64_t>(g.node.size());
   const int64_t bslots = slots / (kTreeBlock / 64);
   int64_t G = cfg_.mult_grid_chunks;
   if (G <= 0) {
@@ -321,16 +391,70 @@ void DeviceMultiEval::set_tree_plans(const TreeGrid& g, bool multT) {
                                  (kMultLds - 16) / static_cast<int64_t>(sizeof(T)), nodes,
                                  static_cast<int>(sizeof(T)), sizeof(T) == 4),
               pm, static_cast<int>(sizeof(T)));
-  if (!multT) return;
-  // multTranspose: chunks, each a wave per data segment
-  TreePlan& pt = tree_multT_[ix];
-  pt.wide = wide;
-  const int64_t batches = (M + 64 * l.kt - 1) / (64 * l.kt);
-  const int64_t per = std::max<int64_t>(kMinNodes, nodes * batches / slots);
-  upload_tree(build_tree_program(g, 1, kMultTEntries, per, 8, sizeof(T) == 4), pt, 8);
 }
 
-bool DeviceMultiEval::set_tree(const TreeGrid& g, bool multT) {
+// multTranspose: chunks; each a wave per data segment, the segments of a chunk
+// by its nodes, so that all waves take about as long (with as many segments for
+// every chunk, 44 % of the wave slots stood idle on a d=10 adaptive grid:
+// 3,030 us against 1,900)
+template <typename T>
+void DeviceMultiEval::set_tree_multT(const TreeGrid& g, int64_t batches) {
+  TreePlan& pt = tree_multT_[sizeof(T) == sizeof(double) ? 0 : 1];
+  const int64_t nodes = static_cast<int64_t>(g.node.size());
+  const int64_t tslots = static_cast<int64_t>(num_cus_) * 16;
+  const int64_t rounds = std::max<int64_t>(
+      2, std::min<int64_t>(6, nodes * batches / (kMultTWork * tslots)));
+  const int64_t per = std::max<int64_t>(kMinNodes, nodes * batches / tslots);
+  const TreeProgram p = build_tree_program(g, 1, kMultTEntries, per, 8, sizeof(T) == 4);
+  upload_tree(p, pt, 8);
+  const double target = cfg_.target_blocks > 0 ? cfg_.target_blocks
+                                               : static_cast<double>(tslots * rounds);
+  const double budget = static_cast<double>(kTreePartialBudget / 8) / static_cast<double>(g.total);
+  double work = 0.0;
+  for (const TreeChunk& c : p.chunks) work += c.nrec + kBatchNodes;
+  std::vector<TreeItem> items;
+  std::vector<TreeSum> sums;
+  int64_t off = 0;
+  pt.segs = 1;
+  for (size_t c = 0; c < p.chunks.size(); ++c) {
+    const TreeChunk& ch = p.chunks[c];
+    int64_t S = cfg_.multT_data_segs;
+    if (S <= 0)
+      S = static_cast<int64_t>(std::min(budget, target * (ch.nrec + kBatchNodes) / work + 0.5));
+    S = std::max<int64_t>(1, std::min<int64_t>(S, batches));
+    const int64_t len = (batches + S - 1) / S;
+    S = (batches + len - 1) / len;
+    pt.segs = std::max<int>(pt.segs, static_cast<int>(S));
+    for (int i = 0; i < ch.n; i += kCols)
+      sums.push_back(TreeSum{std::min(kCols, ch.n - i), static_cast<int>(S), off + i, ch.n,
+                             ch.off0 + i});
+    for (int64_t s = 0; s < S; ++s, off += ch.n)
+      items.push_back(TreeItem{static_cast<int>(c), static_cast<int>(s * len),
+                               static_cast<int>(std::min(batches, (s + 1) * len)), 0, off, 0});
+  }
+  pt.part = static_cast<size_t>(off) * sizeof(double);
+  pt.nitems = static_cast<int>(items.size());
+  pt.nsums = static_cast<int>(sums.size());
+  ensure(&pt.items, &pt.items_cap, items.size() * sizeof(TreeItem));
+  check_hip(hipMemcpy(pt.items, items.data(), items.size() * sizeof(TreeItem),
+                      hipMemcpyHostToDevice),
+            "upload tree items");
+  ensure(&pt.sums, &pt.sums_cap, sums.size() * sizeof(TreeSum));
+  check_hip(hipMemcpy(pt.sums, sums.data(), sums.size() * sizeof(TreeSum), hipMemcpyHostToDevice),
+            "upload tree sums");
+}
+
+int64_t tree_walks(const TreeGrid& g, bool multT) {
+  const int64_t cap = multT ? kMultTEntries : kMultLds / 8;
+  int64_t n = 0;
+  for (const TreeGrid::Node& q : g.node) {
+    const int64_t size = int64_t(1) << q.bits;
+    n += size > cap ? (size + cap - 1) / cap * q.depth : 1;
+  }
+  return n;
+}
+
+bool DeviceMultiEval::set_tree(const TreeGrid& g, bool mult, bool multT) {
   if (g.repeated || g.depth > kTreeMaxDepth || g.node.size() > (size_t(1) << 24)) return false;
   check_hip(hipSetDevice(device_), "hipSetDevice");
   check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
@@ -340,8 +464,8 @@ bool DeviceMultiEval::set_tree(const TreeGrid& g, bool multT) {
   tree_total_ = g.total;
   tree_nodes_ = static_cast<int64_t>(g.node.size());
   tree_depth_ = g.depth;
-  if (serves(Precision::FP64)) set_tree_plans<double>(g, multT);
-  if (serves(Precision::FP32)) set_tree_plans<float>(g, multT);
+  if (serves(Precision::FP64)) set_tree_plans<double>(g, mult, multT);
+  if (serves(Precision::FP32)) set_tree_plans<float>(g, mult, multT);
   return true;
 }
 
@@ -351,12 +475,13 @@ template <typename T>
 void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hipEvent_t* tev,
                                     const MultScratch* ext) {
   hipStream_t s = stream_;
-  const TreePlan& plan = tree_mult_[sizeof(T) == sizeof(double) ? 0 : 1];
+  const int ix = sizeof(T) == sizeof(double) ? 0 : 1;
+  const TreePlan& plan = tree_mult_[ix];
   const TreeLaunch l = basis_ == Basis::ModLinear
-                           ? tree_launch<T, true>(static_cast<int>(D_), tree_depth_, plan.wide)
-                           : tree_launch<T, false>(static_cast<int>(D_), tree_depth_, plan.wide);
-  const int64_t M = static_cast<int64_t>(M_);
-  const unsigned rb = blocks(M, kTreeBlock * l.k);
+                           ? tree_launch<T, true>(static_cast<int>(D_), tree_depth_, tree_wide_[ix])
+                           : tree_launch<T, false>(static_cast<int>(D_), tree_depth_, tree_wide_[ix]);
+  const int64_t nrows = tree_rows_[ix];
+  const unsigned rb = blocks(nrows, kTreeBlock * l.k);
   int G = plan.ngroups, gper = 1;
   // weights in table order first, unless few blocks gather few of them
   const size_t wbytes = (static_cast<size_t>(tree_total_) * sizeof(T) + 255) / 256 * 256;
@@ -367,7 +492,7 @@ void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hip
     check_scratch(*ext, sizeof(T));
     if (wbytes > ext->bytes) weights = false;
     const size_t left = ext->bytes - (weights ? wbytes : 0);
-    const int64_t rows = static_cast<int64_t>(left / (Mpad_ * sizeof(double)));
+    const int64_t rows = static_cast<int64_t>(left / (nrows * sizeof(double)));
     if (rows < G) gper = rows > 1 ? static_cast<int>((G + rows - 1) / rows) : G;
     if (weights) W = static_cast<T*>(ext->base);
     P = reinterpret_cast<double*>(static_cast<unsigned char*>(ext->base) + (weights ? wbytes : 0));
@@ -377,7 +502,7 @@ void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hip
   }
   G = (G + gper - 1) / gper;
   if (G > 1 && !ext) {
-    ensure(&part_, &part_cap_, static_cast<size_t>(G) * Mpad_ * sizeof(double));
+    ensure(&part_, &part_cap_, static_cast<size_t>(G) * nrows * sizeof(double));
     P = static_cast<double*>(part_);
   }
   if (weights) {
@@ -387,9 +512,8 @@ void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hip
     check_hip(hipGetLastError(), "tree weights");
   }
   TreeMultArgs a{};
-  a.X = sizeof(T) == sizeof(double) ? X64_ : X32_;
-  a.ldx = static_cast<int64_t>(Mpad_);
-  a.M = M;
+  a.X = tree_x_[ix];
+  a.ldx = nrows;
   a.D = static_cast<int>(D_);
   a.recs = static_cast<const TreeRec*>(plan.recs);
   a.chunks = static_cast<const TreeChunk*>(plan.chunks);
@@ -401,7 +525,7 @@ void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hip
   a.ti = static_cast<const int32_t*>(tree_ti_);
   a.part = G > 1 ? P : nullptr;
   a.out = d_result;
-  a.dperm = static_cast<const int32_t*>(dperm_);
+  a.sperm = static_cast<const int32_t*>(tree_sperm_[ix]);
   a.zero_off = plan.lds;
   if (tev) check_hip(hipEventRecord(tev[0], s), "hipEventRecord");
   l.mult(a, dim3(rb, static_cast<unsigned>(G)), kTreeBlock, static_cast<unsigned>(plan.lds) + 16, s);
@@ -409,9 +533,8 @@ void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hip
   if (tev) check_hip(hipEventRecord(tev[1], s), "hipEventRecord");
   if (G > 1) {
     clear_launch_error();
-    hipLaunchKernelGGL(reduce_rows_kernel, dim3(blocks(M, kCols)), dim3(kRows * kCols), 0, s, P,
-                       static_cast<int64_t>(Mpad_), G, static_cast<const int32_t*>(dperm_),
-                       static_cast<const double*>(nullptr), d_result, M);
+    hipLaunchKernelGGL(reduce_rows_kernel, dim3(blocks(nrows, kCols)), dim3(kRows * kCols), 0, s,
+                       P, nrows, G, a.sperm, d_result, nrows);
     check_hip(hipGetLastError(), "tree reduce (mult)");
   }
   last_G_ = G;
@@ -420,54 +543,38 @@ void DeviceMultiEval::run_tree_mult(const double* d_alpha, double* d_result, hip
 template <typename T>
 void DeviceMultiEval::run_tree_multT(const double* d_y, double* d_result, hipEvent_t* tev) {
   hipStream_t s = stream_;
-  const TreePlan& plan = tree_multT_[sizeof(T) == sizeof(double) ? 0 : 1];
+  const int ix = sizeof(T) == sizeof(double) ? 0 : 1;
+  const TreePlan& plan = tree_multT_[ix];
   const TreeLaunch l = basis_ == Basis::ModLinear
-                           ? tree_launch<T, true>(static_cast<int>(D_), tree_depth_, plan.wide)
-                           : tree_launch<T, false>(static_cast<int>(D_), tree_depth_, plan.wide);
-  const int64_t M = static_cast<int64_t>(M_), rows = 64 * l.kt;
-  const int64_t batches = (M + rows - 1) / rows;
-  int64_t S = cfg_.multT_data_segs;
-  if (S <= 0) {
-    // two rounds of waves
-    const int waves_cu = basis_ == Basis::ModLinear ? 16 : 12;
-    const int64_t target = cfg_.target_blocks > 0 ? cfg_.target_blocks
-                                                  : 2 * static_cast<int64_t>(num_cus_) * waves_cu;
-    S = std::max<int64_t>(1, target / plan.nchunks);
-    S = std::min<int64_t>(S, std::max<int64_t>(1, kTreePartialBudget / (tree_total_ * 8)));
-  }
-  S = std::min<int64_t>({S, batches, 65535});
-  const int64_t seg = (batches + S - 1) / S * rows;
-  S = (batches * rows + seg - 1) / seg;
+                           ? tree_launch<T, true>(static_cast<int>(D_), tree_depth_, tree_wide_[ix])
+                           : tree_launch<T, false>(static_cast<int>(D_), tree_depth_, tree_wide_[ix]);
   ensure(&Y_, &Y_cap_, Mpad_ * sizeof(T));
-  ensure(&part_, &part_cap_, static_cast<size_t>(S * tree_total_) * sizeof(double));
+  ensure(&part_, &part_cap_, plan.part);
   clear_launch_error();
-  hipLaunchKernelGGL(prep_rows_kernel<T>, dim3(blocks(Mpad_, 256)), dim3(256), 0, s, d_y,
-                     static_cast<const int32_t*>(dperm_), static_cast<T*>(Y_), M,
-                     static_cast<int64_t>(Mpad_));
+  hipLaunchKernelGGL(tree_prep_kernel<T>, dim3(blocks(tree_rows_[ix], 256)), dim3(256), 0, s, d_y,
+                     static_cast<const int32_t*>(tree_sperm_[ix]), static_cast<T*>(Y_),
+                     tree_rows_[ix]);
   check_hip(hipGetLastError(), "tree prep");
   TreeMultTArgs a{};
-  a.X = sizeof(T) == sizeof(double) ? X64_ : X32_;
-  a.ldx = static_cast<int64_t>(Mpad_);
+  a.X = tree_x_[ix];
+  a.ldx = tree_rows_[ix];
   a.D = static_cast<int>(D_);
   a.Y = Y_;
   a.recs = static_cast<const TreeRec*>(plan.recs);
   a.chunks = static_cast<const TreeChunk*>(plan.chunks);
-  a.seg = seg;
-  a.mend = batches * rows;
+  a.items = static_cast<const TreeItem*>(plan.items);
   a.part = static_cast<double*>(part_);
-  a.ntable = tree_total_;
   if (tev) check_hip(hipEventRecord(tev[0], s), "hipEventRecord");
-  l.multT(a, dim3(static_cast<unsigned>(plan.nchunks), static_cast<unsigned>(S)),
-          static_cast<unsigned>(plan.lds), s);
+  l.multT(a, static_cast<unsigned>(plan.nitems), static_cast<unsigned>(plan.lds), s);
   check_hip(hipGetLastError(), "tree multTranspose kernel");
   if (tev) check_hip(hipEventRecord(tev[1], s), "hipEventRecord");
   clear_launch_error();
-  hipLaunchKernelGGL(reduce_rows_kernel, dim3(blocks(tree_total_, kCols)), dim3(kRows * kCols), 0,
-                     s, static_cast<const double*>(part_), tree_total_, static_cast<int>(S),
-                     static_cast<const int32_t*>(tree_ti_),
-                     static_cast<const double*>(nullptr), d_result, tree_total_);
+  hipLaunchKernelGGL(tree_sum_kernel, dim3(static_cast<unsigned>(plan.nsums)), dim3(kRows * kCols),
+                     0, s, static_cast<const double*>(part_),
+                     static_cast<const TreeSum*>(plan.sums),
+                     static_cast<const int32_t*>(tree_ti_), d_result);
   check_hip(hipGetLastError(), "tree reduce (multTranspose)");
-  last_S_ = static_cast<int>(S);
+  last_S_ = plan.segs;
 }
 
 template void DeviceMultiEval::run_tree_mult<double>(const double*, double*, hipEvent_t*,

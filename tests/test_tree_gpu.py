@@ -48,6 +48,28 @@ def loose(d, depth, n, seed):
     return np.ascontiguousarray(a[:, :, 0]), np.ascontiguousarray(a[:, :, 1])
 
 
+@pytest.mark.parametrize("basis", [0, 1])
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("d,top,M", [(3, 5, 1), (3, 5, 255), (6, 4, 1025), (10, 3, 257), (24, 2, 513)])
+def test_equal_points_and_points_by_the_faces(gpu, basis, prec, d, top, M):
+    """All data in one cell (every add meets in one position), then data whose
+    level-1 factors are the smallest, zero or denormal."""
+    capi = gpu
+    print("case", basis, prec, d, top, M, flush=True)
+    lv, ix = capi.Grid(basis, d).regular(top).level_index()
+    rng = np.random.default_rng(M)
+    alpha, y = rng.standard_normal(len(lv)), rng.standard_normal(M)
+    X = np.full((M, d), 0.3125)
+    faces = rng.choice([0.0, 1.0, 1e-310, 1e-40, 2.0 ** -24, 1.0 - 2.0 ** -24, 0.5, 0.3], (M, d))
+    faces = np.where(rng.random((M, d)) < 0.3, faces, rng.random((M, d)))
+    for X in (X, faces.astype(np.float32).astype(np.float64) if prec else faces):
+        op = capi.MultiEval(basis, X, precision=prec).prepare(lv, ix)
+        r, a = op.mult(alpha), op.mult_transpose(y)
+        assert rel(r, oracle.mult(basis, X, lv, ix, alpha)) <= TOL[prec]
+        assert rel(a, oracle.mult_transpose(basis, X, lv, ix, y)) <= TOL[prec]
+        assert np.array_equal(a, op.mult_transpose(y))
+
+
 def grid(capi, basis, kind, d, arg):
     if kind == "regular":
         return capi.Grid(basis, d).regular(arg).level_index()
