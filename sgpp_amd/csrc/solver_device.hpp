@@ -42,13 +42,12 @@ class DeviceRegression {
   void system_mult_host(const double* v, double* q, double lambda, Precision p);
 
  private:
+  void products(const double* v, double* q, Precision p);
   void apply(const double* v, double* q, double lambda, Precision p);
   double dot(const double* x, const double* y);
   void dot_dev(const double* x, const double* y, double* out);
   const double* read_scalars(const double* s, int n);
-  void one_thread(void (*kernel)(double*));
   void axpy(double a, const double* x, double* y);
-  void xpby(const double* x, double b, double* y);
   void sub(const double* x, const double* y, double* z);
   void fill(double* y, double v);
   void copy(const double* x, double* y);

@@ -39,12 +39,6 @@ __global__ void axpy_kernel(double a, const double* __restrict__ x, double* __re
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) y[i] += a * x[i];
 }
-// y = x + b*y
-__global__ void xpby_kernel(const double* __restrict__ x, double b, double* __restrict__ y,
-                            int64_t n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = x[i] + b * y[i];
-}
 // z = x - y
 __global__ void sub_kernel(const double* __restrict__ x, const double* __restrict__ y,
                            double* __restrict__ z, int64_t n) {
@@ -55,33 +49,25 @@ __global__ void fill_kernel(double* __restrict__ y, double v, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) y[i] = v;
 }
-// y += sign * (*a) * x, the step read from device memory
-__global__ void axpy_dev_kernel(double sign, const double* __restrict__ a,
-                                const double* __restrict__ x, double* __restrict__ y, int64_t n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) y[i] += (sign * a[0]) * x[i];
-}
-// y = x + (*b) * y
-__global__ void xpby_dev_kernel(const double* __restrict__ x, const double* __restrict__ b,
-                                double* __restrict__ y, int64_t n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = x[i] + b[0] * y[i];
-}
 // CG scalars in device memory
-enum { kDeltaNew = 0, kDq = 1, kStep = 2, kDeltaOld = 3, kBeta = 4, kNumScalars = 8 };
-// step a = delta_new / (d.q); 0 when d.q == 0 (the host then stops, and the
-// iteration changes no iterate: ConjugateGradients breaks before its update)
-__global__ void cg_step_kernel(double* __restrict__ s) {
-  if (threadIdx.x == 0) s[kStep] = s[kDq] != 0.0 ? s[kDeltaNew] / s[kDq] : 0.0;
-}
-__global__ void cg_keep_delta_kernel(double* __restrict__ s) {
-  if (threadIdx.x == 0) s[kDeltaOld] = s[kDeltaNew];
-}
-__global__ void cg_beta_kernel(double* __restrict__ s) {
-  if (threadIdx.x == 0) s[kBeta] = s[kDeltaNew] / s[kDeltaOld];
-}
+enum { kDeltaNew = 0, kDq = 1, kDeltaOld = 2, kNumScalars = 8 };
 
-// stage 1: block b sums the contiguous chunk [b*chunk, (b+1)*chunk)
+// The sum of v over a block's threads, in a fixed order, in every thread.
+__device__ __forceinline__ double block_sum(double v, double* s) {
+  s[threadIdx.x] = v;
+  __syncthreads();
+  for (int w = kRB / 2; w > 0; w >>= 1) {
+    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    __syncthreads();
+  }
+  const double sum = s[0];
+  __syncthreads();
+  return sum;
+}
+// A dot product in two stages: block b sums the contiguous chunk
+// [b*chunk, (b+1)*chunk) into part[b]; the kDotBlocks parts are then added by
+// one block, or by every block of the kernel that uses the sum.
+static_assert(kDotBlocks == kRB, "one part per thread");
 __global__ __launch_bounds__(kRB) void dot_stage1(const double* __restrict__ x,
                                                   const double* __restrict__ y, int64_t n,
                                                   int64_t chunk, double* __restrict__ part) {
@@ -90,26 +76,83 @@ __global__ __launch_bounds__(kRB) void dot_stage1(const double* __restrict__ x,
   const int64_t b1 = min(b0 + chunk, n);
   double acc = 0.0;
   for (int64_t i = b0 + threadIdx.x; i < b1; i += kRB) acc += x[i] * y[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = kRB / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+  acc = block_sum(acc, s);
+  if (threadIdx.x == 0) part[blockIdx.x] = acc;
 }
-__global__ __launch_bounds__(kRB) void dot_stage2(const double* __restrict__ part, int nb,
+__global__ __launch_bounds__(kRB) void dot_stage2(const double* __restrict__ part,
                                                   double* __restrict__ out) {
   __shared__ double s[kRB];
+  const double sum = block_sum(part[threadIdx.x], s);
+  if (threadIdx.x == 0) out[0] = sum;
+}
+
+// A CG iteration between two products, in three kernels (as ten, launches and
+// round trips of 2-4 us each took a third of the iterations of a d=6 level-5 solve:
+// 7.6 to 6.7 ms). The sums are those of dot_stage1 and dot_stage2, in their order.
+// 1: q += lambda_m * d; part_dq = d . q by chunks
+__global__ __launch_bounds__(kRB) void cg_dq_kernel(const double* __restrict__ d, double lambda_m,
+                                                    double* __restrict__ q, int64_t n,
+                                                    int64_t chunk, double* __restrict__ part_dq) {
+  __shared__ double s[kRB];
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * chunk;
+  const int64_t b1 = min(b0 + chunk, n);
   double acc = 0.0;
-  for (int i = threadIdx.x; i < nb; i += kRB) acc += part[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = kRB / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
+  for (int64_t i = b0 + threadIdx.x; i < b1; i += kRB) {
+    const double v = q[i] + lambda_m * d[i];
+    q[i] = v;
+    acc += d[i] * v;
   }
-  if (threadIdx.x == 0) out[0] = s[0];
+  acc = block_sum(acc, s);
+  if (threadIdx.x == 0) part_dq[blockIdx.x] = acc;
+}
+// 2: the step a = delta_new / (d.q), 0 when d.q == 0 (the host then stops, and the
+// iteration changes no iterate: ConjugateGradients breaks before its update);
+// x += a d; with r, r -= a q and part_rr = r . r by chunks
+__global__ __launch_bounds__(kRB) void cg_step_kernel(const double* __restrict__ part_dq,
+                                                      double* __restrict__ scal,
+                                                      const double* __restrict__ d,
+                                                      const double* __restrict__ q,
+                                                      double* __restrict__ x,
+                                                      double* __restrict__ r, int64_t n,
+                                                      int64_t chunk,
+                                                      double* __restrict__ part_rr) {
+  __shared__ double s[kRB];
+  const double dq = block_sum(part_dq[threadIdx.x], s);
+  const double delta = scal[kDeltaNew];  // (not written here)
+  const double a = dq != 0.0 ? delta / dq : 0.0;
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * chunk;
+  const int64_t b1 = min(b0 + chunk, n);
+  double acc = 0.0;
+  for (int64_t i = b0 + threadIdx.x; i < b1; i += kRB) {
+    x[i] += a * d[i];
+    if (r) {
+      const double v = r[i] + (-a) * q[i];
+      r[i] = v;
+      acc += v * v;
+    }
+  }
+  if (r) {
+    acc = block_sum(acc, s);
+    if (threadIdx.x == 0) part_rr[blockIdx.x] = acc;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scal[kDq] = dq;
+    scal[kDeltaOld] = delta;
+  }
+}
+// 3: delta_new = r . r, beta = delta_new / delta_old, d = r + beta d
+__global__ __launch_bounds__(kRB) void cg_direction_kernel(const double* __restrict__ part_rr,
+                                                           double* __restrict__ scal,
+                                                           const double* __restrict__ r,
+                                                           double* __restrict__ d, int64_t n,
+                                                           int64_t chunk) {
+  __shared__ double s[kRB];
+  const double rr = block_sum(part_rr[threadIdx.x], s);
+  const double beta = rr / scal[kDeltaOld];
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * chunk;
+  const int64_t b1 = min(b0 + chunk, n);
+  for (int64_t i = b0 + threadIdx.x; i < b1; i += kRB) d[i] = r[i] + beta * d[i];
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[kDeltaNew] = rr;
 }
 
 unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + kRB - 1) / kRB); }
@@ -123,7 +166,7 @@ DeviceRegression::DeviceRegression(DeviceMultiEval& op) : op_(op) {
   const size_t nvec = 9;
   check_hip(hipMalloc(&vec_, nvec * N_ * sizeof(double)), "hipMalloc(solver vectors)");
   check_hip(hipMalloc(&tempM_, M_ * sizeof(double)), "hipMalloc(solver temp)");
-  check_hip(hipMalloc(&dotpart_, (kDotBlocks + 1 + kNumScalars) * sizeof(double)),
+  check_hip(hipMalloc(&dotpart_, (2 * kDotBlocks + 1 + kNumScalars) * sizeof(double)),
             "hipMalloc(dot)");
   check_hip(hipHostMalloc(&hostscal_, kNumScalars * sizeof(double)), "hipHostMalloc");
   alpha_ = static_cast<double*>(vec_);
@@ -135,7 +178,7 @@ DeviceRegression::DeviceRegression(DeviceMultiEval& op) : op_(op) {
   w_ = c_ + N_;
   corr_ = w_ + N_;
   rhs_ = corr_ + N_;
-  scal_ = static_cast<double*>(dotpart_) + kDotBlocks + 1;
+  scal_ = static_cast<double*>(dotpart_) + 2 * kDotBlocks + 1;
 }
 
 DeviceRegression::~DeviceRegression() {
@@ -146,17 +189,19 @@ DeviceRegression::~DeviceRegression() {
   if (hostscal_) (void)hipHostFree(hostscal_);
 }
 
-void DeviceRegression::apply(const double* v, double* q, double lambda, Precision p) {
+// q = B^T B v
+void DeviceRegression::products(const double* v, double* q, Precision p) {
   op_.mult_device(v, tempM_, p);
   op_.mult_transpose_device(tempM_, q, p);
-  clear_launch_error();
-  hipLaunchKernelGGL(axpy_kernel, dim3(blocks_for(N_)), dim3(kRB), 0, op_.stream(),
-                     static_cast<double>(M_) * lambda, v, q, static_cast<int64_t>(N_));
-  check_hip(hipGetLastError(), "axpy");
   if (p == Precision::FP64)
     ++fp64_matvecs_;
   else
     ++fp32_matvecs_;
+}
+
+void DeviceRegression::apply(const double* v, double* q, double lambda, Precision p) {
+  products(v, q, p);
+  axpy(static_cast<double>(M_) * lambda, v, q);
 }
 
 // x . y into device memory (out), fixed-order two-stage reduction
@@ -167,7 +212,7 @@ void DeviceRegression::dot_dev(const double* x, const double* y, double* out) {
   clear_launch_error();
   hipLaunchKernelGGL(dot_stage1, dim3(kDotBlocks), dim3(kRB), 0, op_.stream(), x, y, n, chunk,
                      part);
-  hipLaunchKernelGGL(dot_stage2, dim3(1), dim3(kRB), 0, op_.stream(), part, kDotBlocks, out);
+  hipLaunchKernelGGL(dot_stage2, dim3(1), dim3(kRB), 0, op_.stream(), part, out);
   check_hip(hipGetLastError(), "dot");
 }
 
@@ -180,15 +225,9 @@ const double* DeviceRegression::read_scalars(const double* s, int n) {
 }
 
 double DeviceRegression::dot(const double* x, const double* y) {
-  double* out = static_cast<double*>(dotpart_) + kDotBlocks;
+  double* out = static_cast<double*>(dotpart_) + 2 * kDotBlocks;
   dot_dev(x, y, out);
   return read_scalars(out, 1)[0];
-}
-
-void DeviceRegression::one_thread(void (*kernel)(double*)) {
-  clear_launch_error();
-  hipLaunchKernelGGL(kernel, dim3(1), dim3(64), 0, op_.stream(), scal_);
-  check_hip(hipGetLastError(), "cg scalars");
 }
 
 void DeviceRegression::axpy(double a, const double* x, double* y) {
@@ -196,12 +235,6 @@ void DeviceRegression::axpy(double a, const double* x, double* y) {
   hipLaunchKernelGGL(axpy_kernel, dim3(blocks_for(N_)), dim3(kRB), 0, op_.stream(), a, x, y,
                      static_cast<int64_t>(N_));
   check_hip(hipGetLastError(), "axpy");
-}
-void DeviceRegression::xpby(const double* x, double b, double* y) {
-  clear_launch_error();
-  hipLaunchKernelGGL(xpby_kernel, dim3(blocks_for(N_)), dim3(kRB), 0, op_.stream(), x, b, y,
-                     static_cast<int64_t>(N_));
-  check_hip(hipGetLastError(), "xpby");
 }
 void DeviceRegression::sub(const double* x, const double* y, double* z) {
   clear_launch_error();
@@ -248,32 +281,29 @@ size_t DeviceRegression::cg(double* x, const double* rhs, double lambda, Precisi
   if (!reuse) delta0 = delta_new * eps2;
   if (start_delta) *start_delta = reuse ? delta0 / eps2 : delta_new;
   size_t it = 0;
-  const unsigned nb = blocks_for(N_);
   const int64_t n = static_cast<int64_t>(N_);
+  const int64_t chunk = (n + kDotBlocks - 1) / kDotBlocks;
+  double* part_dq = static_cast<double*>(dotpart_);
+  double* part_rr = part_dq + kDotBlocks;
+  hipStream_t s = op_.stream();
   while (it < max_it && delta_new > delta0) {
-    apply(d_, q_, lambda, p);
-    dot_dev(d_, q_, scal_ + kDq);
-    one_thread(cg_step_kernel);
+    products(d_, q_, p);
+    const bool replace = (it % 50) == 0 && it > 0;  // the true residual
     clear_launch_error();
-    hipLaunchKernelGGL(axpy_dev_kernel, dim3(nb), dim3(kRB), 0, op_.stream(), 1.0,
-                       scal_ + kStep, d_, x, n);
-    check_hip(hipGetLastError(), "axpy");
-    if ((it % 50) == 0 && it > 0) {
+    hipLaunchKernelGGL(cg_dq_kernel, dim3(kDotBlocks), dim3(kRB), 0, s, d_,
+                       static_cast<double>(M_) * lambda, q_, n, chunk, part_dq);
+    hipLaunchKernelGGL(cg_step_kernel, dim3(kDotBlocks), dim3(kRB), 0, s, part_dq, scal_, d_, q_,
+                       x, replace ? nullptr : r_, n, chunk, part_rr);
+    check_hip(hipGetLastError(), "cg step");
+    if (replace) {
       apply(x, w_, lambda, p);
       sub(rhs, w_, r_);
-    } else {
       clear_launch_error();
-      hipLaunchKernelGGL(axpy_dev_kernel, dim3(nb), dim3(kRB), 0, op_.stream(), -1.0,
-                         scal_ + kStep, q_, r_, n);
-      check_hip(hipGetLastError(), "axpy");
+      hipLaunchKernelGGL(dot_stage1, dim3(kDotBlocks), dim3(kRB), 0, s, r_, r_, n, chunk, part_rr);
     }
-    one_thread(cg_keep_delta_kernel);
-    dot_dev(r_, r_, scal_ + kDeltaNew);
-    one_thread(cg_beta_kernel);
-    clear_launch_error();
-    hipLaunchKernelGGL(xpby_dev_kernel, dim3(nb), dim3(kRB), 0, op_.stream(), r_,
-                       scal_ + kBeta, d_, n);
-    check_hip(hipGetLastError(), "xpby");
+    hipLaunchKernelGGL(cg_direction_kernel, dim3(kDotBlocks), dim3(kRB), 0, s, part_rr, scal_, r_,
+                       d_, n, chunk);
+    check_hip(hipGetLastError(), "cg direction");
     // d.q and delta_new (kDeltaNew = 0, kDq = 1): one synchronisation per
     // iteration. d.q == 0 stops before the count (the reference's break);
     // the step was 0, so x is unchanged.
