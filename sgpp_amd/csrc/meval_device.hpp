@@ -96,7 +96,9 @@ class DeviceMultiEval {
   DeviceMultiEval(const DeviceMultiEval&) = delete;
   DeviceMultiEval& operator=(const DeviceMultiEval&) = delete;
 
-  // level/index: N x d row-major uint32 (the grid storage's point order).
+  // level/index: N x d row-major uint32 (the grid storage's point order). A
+  // refused grid leaves the one before it; a call that fails later (memory)
+  // leaves none.
   void set_grid(const uint32_t* level, const uint32_t* index, size_t N);
 
   // Device-pointer entry points (inputs/outputs already in HBM, FP64).

@@ -373,11 +373,15 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   }
   std::vector<double> li0, sc0;
   encode_grid(basis_, D_, N, level, index, li0, sc0);
-  N_ = N;
-  Npad_ = ((N + kGridPad - 1) / kGridPad) * kGridPad;
   TreeGrid tg;
-  if (set_paths(build_tree_grid(D_, N, level, index, true, tg) ? &tg : nullptr, li0, pmask))
+  const bool tree = build_tree_grid(D_, N, level, index, true, tg);
+  const size_t Npad = ((N + kGridPad - 1) / kGridPad) * kGridPad;
+  N_ = 0;  // (set when the grid is laid out whole)
+  if (set_paths(tree ? &tg : nullptr, li0, pmask)) {
+    N_ = N;
+    Npad_ = Npad;
     return;
+  }
   // storage order: by the set of non-constant dimensions, then by the Morton
   // code of the support's centre, so that a 64-point tile holds points with
   // the same dimensions in a small region
@@ -388,7 +392,6 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
     for (size_t e = 0; e < D_ * 2; ++e) li[s * D_ * 2 + e] = li0[j * D_ * 2 + e];
     sc[s] = sc0[j];
   }
-  const size_t Npad = ((N + kGridPad - 1) / kGridPad) * kGridPad;
   // padded points: (L, I) = (1, 4) in every dimension, a factor that is
   // exactly 0 on [0, 1] (u = x - 4), so the culling tests drop them; weight 0
   // through A, rows ignored by the reductions
@@ -403,7 +406,6 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   std::vector<uint32_t> pm(Npad, 0u);
   for (size_t s = 0; s < N; ++s) pm[s] = pmask[order[s]];
   check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-  N_ = N;
   Npad_ = Npad;
   ensure(&pm_, &pm_cap_, Npad_ * sizeof(uint32_t));
   check_hip(hipMemcpy(pm_, pm.data(), Npad_ * sizeof(uint32_t), hipMemcpyHostToDevice),
@@ -411,15 +413,15 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   ensure(reinterpret_cast<void**>(&scale_), &gridcap_scale_, Npad_ * sizeof(double));
   check_hip(hipMemcpy(scale_, sc.data(), Npad_ * sizeof(double), hipMemcpyHostToDevice),
             "upload scale");
-  ensure(&perm_, &perm_cap_, N_ * sizeof(int32_t));
-  check_hip(hipMemcpy(perm_, order.data(), N_ * sizeof(int32_t), hipMemcpyHostToDevice),
+  ensure(&perm_, &perm_cap_, N * sizeof(int32_t));
+  check_hip(hipMemcpy(perm_, order.data(), N * sizeof(int32_t), hipMemcpyHostToDevice),
             "upload permutation");
   if (serves(Precision::FP64)) {
     ensure(&LI64_, &gridcap_li64_, li.size() * sizeof(double));
     check_hip(hipMemcpy(LI64_, li.data(), li.size() * sizeof(double), hipMemcpyHostToDevice),
               "upload LI64");
     // FP32 boxes of the FP64 supports, rounded outwards
-    const std::vector<float> tb = tile_boxes<float>(li, Npad_, N_, D_);
+    const std::vector<float> tb = tile_boxes<float>(li, Npad_, N, D_);
     ensure(&TB64_, &tbcap64_, tb.size() * sizeof(float));
     check_hip(hipMemcpy(TB64_, tb.data(), tb.size() * sizeof(float), hipMemcpyHostToDevice),
               "upload tile boxes");
@@ -431,11 +433,12 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
               "upload LI32");
     // boxes of the FP32 (L, I) the FP32 kernels evaluate
     const std::vector<double> l32d(l32.begin(), l32.end());
-    const std::vector<float> tb = tile_boxes<float>(l32d, Npad_, N_, D_);
+    const std::vector<float> tb = tile_boxes<float>(l32d, Npad_, N, D_);
     ensure(&TB32_, &tbcap32_, tb.size() * sizeof(float));
     check_hip(hipMemcpy(TB32_, tb.data(), tb.size() * sizeof(float), hipMemcpyHostToDevice),
               "upload tile boxes");
   }
+  N_ = N;
   if (D_ <= static_cast<size_t>(kMaxTemplD) && !count_) {
     if (serves(Precision::FP64))
       choose_mult_order<double>(static_cast<const double*>(X64_),
@@ -587,6 +590,7 @@ void DeviceMultiEval::choose_mult_order(const T* X, const T* LI, const float* TB
     }
   } catch (...) {
     mult_cf_[ix] = multT_cf_[ix] = 0;
+    N_ = 0;
     release();
     throw;
   }

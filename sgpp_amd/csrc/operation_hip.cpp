@@ -46,8 +46,8 @@ OperationMultiEvalHIP::~OperationMultiEvalHIP() {}
 void OperationMultiEvalHIP::prepare() {
   std::vector<uint32_t> level, index;
   grid.getStorage().getLevelIndexArrays(level, index);
+  dev_->set_grid(level.data(), index.data(), grid.getSize());
   numGrid_ = grid.getSize();
-  dev_->set_grid(level.data(), index.data(), numGrid_);
   isPrepared = true;
 }
 

@@ -358,6 +358,7 @@ void DeviceMultiEval::set_grid_subspace(const uint32_t* level, const uint32_t* i
     for (; d < D_; ++d) steps += !(basis_ == Basis::ModLinear && lv[s][d] == 1);
   }
   if (nchunk > 65535) throw input_error("too many subspace chunks for one launch");
+  N_ = 0;  // (set when the grid is laid out whole)
   if (set_paths(&tg, {}, {})) {
     N_ = N;
     Npad_ = N;
@@ -386,7 +387,6 @@ void DeviceMultiEval::set_grid_subspace(const uint32_t* level, const uint32_t* i
   }
   if (chunks.size() > 65535) throw input_error("too many subspace chunks for one launch");
   check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-  N_ = N;
   Npad_ = N;
   nchunk_ = static_cast<int>(chunks.size());
   nsub_ = nsub;
@@ -420,6 +420,7 @@ void DeviceMultiEval::set_grid_subspace(const uint32_t* level, const uint32_t* i
   check_hip(hipMemcpy(sub_chunk_, chunks.data(), chunks.size() * sizeof(SubChunk),
                       hipMemcpyHostToDevice),
             "upload subspace chunks");
+  N_ = N;
 }
 
 void DeviceMultiEval::run_subspace_mult(const double* d_alpha, double* d_result, hipEvent_t* tev) {

@@ -1,0 +1,65 @@
+"""Preparing a grid, on host memory: what a failed call leaves, and what a grid's layout takes."""
+import pytest
+
+from host_hip import on_host  # noqa: F401
+
+
+@pytest.mark.parametrize("algorithm", [0, 1])
+@pytest.mark.parametrize("basis", [0, 1])
+def test_failed_prepare_leaves_no_grid(on_host, algorithm, basis):
+    """Whichever allocation fails, no product runs on what the call left behind, and the
+    next prepare works."""
+    out = on_host("""
+        X = workloads.uniform_points(1, 500, 3)
+        small = capi.Grid(%d, 3).regular(2).level_index()
+        large = capi.Grid(%d, 3).regular(6).level_index()
+        failed = 0
+        for first, then in ((None, large), (small, large), (large, small)):
+            for after in range(30):
+                op = capi.MultiEval(%d, X, algorithm=%d)
+                if first is not None:
+                    op.prepare(*first)
+                launches()
+                hip.host_hip_fail_malloc(after, 1)
+                try:
+                    op.prepare(*then)
+                    ok = True
+                except capi.SGppHIPError:
+                    ok = False
+                hip.host_hip_fail_malloc(-1, 0)
+                if ok:
+                    continue
+                failed += 1
+                launches()
+                op.N = capi.F["sgpp_hip_meval_num_grid"](op.h)
+                for call, n in ((op.mult, op.N), (op.mult_transpose, len(X))):
+                    try:
+                        call(np.zeros(n))
+                    except capi.SGppHIPError as e:
+                        assert "grid not set" in str(e), e
+                    else:
+                        raise AssertionError("a product ran after a failed prepare")
+                assert launches() == []
+                op.prepare(*small).mult(np.zeros(len(small[0])))
+                assert launches()
+        print(failed)
+    """ % (basis, basis, basis, algorithm))
+    assert int(out) > 0
+
+
+def test_refused_grid_leaves_the_old_one(on_host):
+    on_host("""
+        X = workloads.uniform_points(1, 500, 3)
+        lv, ix = capi.Grid(0, 3).regular(3).level_index()
+        for algorithm in (0, 1):
+            op = capi.MultiEval(0, X, algorithm=algorithm).prepare(lv, ix)
+            bad = ix.copy()
+            bad[0] = 2
+            try:
+                op.prepare(lv[:5], bad[:5])
+                raise AssertionError("accepted")
+            except capi.SGppHIPError as e:
+                assert e.status_name == "INVALID_ARGUMENT"
+            assert capi.F["sgpp_hip_meval_num_grid"](op.h) == len(lv)
+            op.mult(np.zeros(len(lv)))
+    """)
