@@ -200,6 +200,7 @@ class DeviceMultiEval {
     int lds = 0;  // bytes of the largest chunk's tables
   };
   bool set_tree(const TreeGrid& g, bool mult, bool multT);
+  void release_tree();  // frees the walks' buffers
   // Kernels that evaluate a direction: the algorithm's own or the
   // subspace tree's
   enum class Path { Own, Tree };

@@ -327,12 +327,10 @@ DeviceMultiEval::~DeviceMultiEval() {
   void* bufs[] = {X64_,   X32_,   WB64_,  WB32_,  LI64_,    LI32_,   TB64_,
                   TB32_,  scale_, perm_,  pm_,    dperm_,   A_,      Y_,
                   part_,  hin_,   hout_,  sub_desc_, sub_ti_, sub_te_, sub_tw_,
-                  sub_chunk_, tree_ti_, tree_x_[0], tree_x_[1], tree_sperm_[0], tree_sperm_[1]};
+                  sub_chunk_};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
-  for (TreePlan* p : {&tree_mult_[0], &tree_mult_[1], &tree_multT_[0], &tree_multT_[1]})
-    for (void* b : {p->recs, p->chunks, p->groups, p->items, p->sums})
-      if (b) (void)hipFree(b);
+  release_tree();
   for (auto* pool : {&tm_mult_, &tm_multT_})
     for (auto& e : *pool) {
       (void)hipEventDestroy(e.a);
@@ -503,10 +501,17 @@ bool DeviceMultiEval::set_paths(const TreeGrid* tree, const std::vector<double>&
     mult = cost > t.mult * static_cast<double>(wm);
     multT = cost > t.multT * static_cast<double>(wt);
   }
-  if ((mult || multT) && set_tree(*tree, mult, multT)) {
-    if (mult) mult_path_ = Path::Tree;
-    if (multT) multT_path_ = Path::Tree;
+  if (!mult && !multT) return false;
+  try {
+    if (!set_tree(*tree, mult, multT)) return false;
+  } catch (const device_error&) {
+    // no memory for the walks' copy of the data, tables and programs (up to
+    // three times the data): the other kernels need none of it
+    release_tree();
+    return false;
   }
+  if (mult) mult_path_ = Path::Tree;
+  if (multT) multT_path_ = Path::Tree;
   return mult_path_ != Path::Own && multT_path_ != Path::Own;
 }
 

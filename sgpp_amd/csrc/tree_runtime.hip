@@ -469,6 +469,27 @@ bool DeviceMultiEval::set_tree(const TreeGrid& g, bool mult, bool multT) {
   return true;
 }
 
+void DeviceMultiEval::release_tree() {
+  (void)hipStreamSynchronize(stream_);
+  auto drop = [](void** buf, size_t* cap) {
+    if (*buf) (void)hipFree(*buf);
+    *buf = nullptr;
+    *cap = 0;
+  };
+  drop(&tree_ti_, &tree_ti_cap_);
+  for (int ix = 0; ix < 2; ++ix) {
+    drop(&tree_x_[ix], &tree_x_cap_[ix]);
+    drop(&tree_sperm_[ix], &tree_sperm_cap_[ix]);
+    for (TreePlan* p : {&tree_mult_[ix], &tree_multT_[ix]}) {
+      drop(&p->recs, &p->recs_cap);
+      drop(&p->chunks, &p->chunks_cap);
+      drop(&p->groups, &p->groups_cap);
+      drop(&p->items, &p->items_cap);
+      drop(&p->sums, &p->sums_cap);
+    }
+  }
+}
+
 // ---------------------------------------------------------------- launches
 
 template <typename T>

@@ -63,3 +63,30 @@ def test_refused_grid_leaves_the_old_one(on_host):
             assert capi.F["sgpp_hip_meval_num_grid"](op.h) == len(lv)
             op.mult(np.zeros(len(lv)))
     """)
+
+
+@pytest.mark.parametrize("algorithm", [0, 1])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_no_memory_for_the_walks(on_host, algorithm, precision):
+    """A grid that its algorithm's own kernels can evaluate is not refused because one of
+    the walks' buffers could not be allocated."""
+    if algorithm == 1 and precision == 1:
+        pytest.skip("not a subspace operator")
+    out = on_host("""
+        X = workloads.uniform_points(1, 500, 3)
+        lv, ix = capi.Grid(0, 3).regular(5).level_index()
+        own = 0
+        for after in range(20):
+            op = capi.MultiEval(0, X, precision=%d, algorithm=%d)
+            hip.host_hip_fail_malloc(after, 0)
+            op.prepare(lv, ix)
+            hip.host_hip_fail_malloc(-1, 0)
+            launches()
+            op.mult(np.zeros(len(lv)))
+            op.mult_transpose(np.zeros(len(X)))
+            own += not any("tree" in name for name, _, _, _ in launches())
+            op.prepare(lv, ix).mult(np.zeros(len(lv)))
+            assert any("tree" in name for name, _, _, _ in launches())
+        print(own)
+    """ % (precision, algorithm))
+    assert int(out) >= 5
