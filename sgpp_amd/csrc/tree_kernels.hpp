@@ -110,8 +110,13 @@ __device__ __forceinline__ void dim_values(const DimRegs<T, DB> (&v)[K], int r, 
   dim_values<T, DB, K, 1>(vs, r, outs);
 }
 
+// Linear grids walked with the dimensions passed (kTreePassDims)
+template <int DB, bool kMod>
+constexpr bool kTreePass = !kMod && DB > 0 && DB <= kTreePassDims;
+
 // The data points of a walk, as tree_points_kernel stores them: per dimension
-// the coordinate times 2^32 and, for Linear grids, 2 over the level-1 factor, in
+// the coordinate times 2^32 and, for Linear grids, 2^D times the product of the later
+// dimensions' halved level-1 factors (kTreePass) or 2 over the level-1 factor, in
 // registers (DB > 0) or, for many dimensions (DB == 0), read from memory when a
 // run begins; and the product of all level-1 factors.
 template <typename T, int DB, int K, bool kMod>
@@ -131,11 +136,10 @@ struct TreePoints {
       }
     }
   }
+  __device__ __forceinline__ void coordinates(int r, T (&xr)[K]) const { dim_values(x, r, xr); }
   __device__ __forceinline__ void values(int r, T (&xr)[K], T (&cr)[K]) const {
     if constexpr (kMod) {
-      const DimRegs<T, DB>(*const v[1])[K] = {&x};
-      T(*const out[1])[K] = {&xr};
-      dim_values<T, DB, K, 1>(v, r, out);
+      coordinates(r, xr);
     } else {
       const DimRegs<T, DB>(*const v[2])[K] = {&x, &c};
       T(*const out[2])[K] = {&xr, &cr};
@@ -172,8 +176,11 @@ struct TreePoints<T, 0, K, kMod> {
 // and rr, twice the product of all factors but the run's own. Per node and
 // data point, with v = 2^(l-1) x (its cells are the unit intervals):
 //   Linear: half the hat is |v - rint(v)|, the distance to the nearest cell
-//     edge (exact); R times 2 over the dimension's level-1 factor takes that
-//     factor out.
+//     edge (exact). With kTreePass R is the product of the halved factors of the
+//     dimensions up to the subspace's last refined one, extended at a run by those
+//     it passes, and rr R times the product of the later ones (which holds the
+//     halves' 2^D); otherwise R times 2 over the dimension's level-1 factor
+//     takes that factor out.
 //   ModLinear: level-1 factors are 1. The extrapolated boundary functions are
 //     2 - 2^l min(x, 1-x), which exceeds the hat in the boundary cells only:
 //     the larger of the two.
@@ -187,7 +194,7 @@ struct TreeWalk {
   T xr[K], cr[K], rr[K];
   unsigned fx[K];
 
-  __device__ __forceinline__ void run(TreeRecPtr recs, const T (&R0)[K]) {
+  __device__ __forceinline__ void run(TreeRecPtr recs, T (&R0)[K]) {
     next = recs;
     cur = next[0];
     unsigned F0[K];
@@ -196,14 +203,24 @@ struct TreeWalk {
     level<0>(R0, F0);
   }
 
+  static constexpr bool kPass = kTreePass<DB, kMod>;
   template <int kDepth>
-  __device__ __forceinline__ void level(const T (&R)[K], const unsigned (&F)[K]) {
+  __device__ __forceinline__ void level(T (&R)[K], const unsigned (&F)[K]) {
     for (;;) {
       const unsigned off = cur.x, ctl = cur.y, scale = cur.z;
       ++next;
       cur = next[0];  // in flight during this node
       if (ctl & kTreeRun) {
-        pts.values((ctl >> kTreeDimShift) & 63u, xr, cr);
+        const int r = (ctl >> kTreeDimShift) & 63u;
+        if constexpr (kPass)
+          for (int d = r - static_cast<int>((ctl >> kTreePassShift) & 15u); d < r; ++d) {
+            T h[K];
+            pts.coordinates(d, h);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+              R[k] *= min_raw(h[k], T(4294967296.0) - h[k]) * T(0x1.0p-32);
+          }
+        pts.values(r, xr, cr);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           fx[k] = to_fixed(xr[k]);
@@ -216,18 +233,24 @@ struct TreeWalk {
       for (int k = 0; k < K; ++k) E[k] = __builtin_amdgcn_alignbit(F[k], fx[k], ctl);
       use.begin(off, ctl, E);
       const T L = scale_of(scale, T(0));
-      T P[K];
+      T P[K], e[K];
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         const T v = xr[k] * L;
-        const T e = v - rint_raw(v);
-        P[k] = rr[k] * (kMod ? max_abs(e, fmaT(-L, cr[k], T(1))) : absT(e));
+        e[k] = v - rint_raw(v);
+        P[k] = rr[k] * (kMod ? max_abs(e[k], fmaT(-L, cr[k], T(1))) : absT(e[k]));
       }
       use.end(off, ctl, P, E);
       if (ctl & (kTreePush | kTreeLast | kTreeFlush)) {
         if (sizeof(T) == 4 && (ctl & kTreeFlush)) use.flush();
         if constexpr (kDepth + 1 < MD)
-          if (ctl & kTreePush) level<kDepth + 1>(P, E);
+          if (ctl & kTreePush) {
+            if constexpr (kPass) {
+#pragma unroll
+              for (int k = 0; k < K; ++k) P[k] = R[k] * absT(e[k]);
+            }
+            level<kDepth + 1>(P, E);
+          }
         if (ctl & kTreeLast) return;
       }
     }
@@ -281,10 +304,11 @@ struct TreeGather {
 // (one scalar instruction issues in four cycles, so several points per lane share
 // a node's). The weights of a chunk's subspaces are gathered from LDS, where up to
 // 64 cells meet no bank conflict. Kernel times against the culled kernels: Linear
-// d=8 level 6, 5e5 points, FP32 1,179 to 246 us, FP64 1,678 to 378; d=20 adaptive,
+// d=8 level 6, 5e5 points, FP32 1,179 to 260 us, FP64 1,678 to 403; d=20 adaptive,
 // 5e5 points, FP32 6,523 to 3,023; ModLinear d=10 adaptive, 1e6 points, FP32 2,051
-// to 1,403. Factors relative to the level-1 ones, instead of extending each product
-// by the dimensions passed: d=20 4,960 to 3,020, d=8 284 to 246 us.
+// to 1,403. Taking level-1 factors out, instead of passing dimensions: d=20 4,960 to
+// 3,020 us; d=8 260 to 230, but with a larger error than the culled kernels'
+// (kTreePassDims).
 template <typename T, int DB, int K, bool kMod, int MD>
 __global__ __launch_bounds__(kTreeBlock) __attribute__((amdgpu_waves_per_eu(kMod ? 4 : 3)))
 void tree_mult_kernel(const TreeMultArgs a) {
@@ -328,7 +352,10 @@ void tree_mult_kernel(const TreeMultArgs a) {
     }
     if (ch.nrec > 0) {
       TreeWalk<T, DB, K, kMod, MD, TreeGather<T, K>> walk{pts, g, nullptr, TreeRecWords{}};
-      walk.run((TreeRecPtr)(a.recs + ch.rec0), all);
+      T start[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) start[k] = kTreePass<DB, kMod> ? T(1) : all[k];
+      walk.run((TreeRecPtr)(a.recs + ch.rec0), start);
       g = walk.use;
       g.flush();
     }
@@ -403,7 +430,7 @@ struct TreeScatter {
 
 // Bound by vector instructions, the LDS adds about half of the time beside them.
 // Kernel times against the culled kernel: Linear d=8 level 6, 5e5 points, FP32
-// 1,621 to 469 us, FP64 2,300 to 574; ModLinear d=10 adaptive, 1e6 points, FP32
+// 1,621 to 515 us, FP64 2,300 to 579; ModLinear d=10 adaptive, 1e6 points, FP32
 // 2,218 to 1,903; against the subspace algorithm's own, d=7 level 6, 2.5e5 points,
 // 681 to 224 with the final sums.
 template <typename T, int DB, int K, bool kMod, int MD>
@@ -426,11 +453,14 @@ void tree_multT_kernel(const TreeMultTArgs a) {
     for (int k = 0; k < K; ++k) y[k] = static_cast<const T*>(a.Y)[m + k * 64];
     pts.load(static_cast<const T*>(a.X), a.ldx, a.D, m, all);
 #pragma unroll
-    for (int k = 0; k < K; ++k) y[k] *= all[k];
+    for (int k = 0; k < K; ++k) {
+      all[k] *= y[k];
+      if constexpr (!kTreePass<DB, kMod>) y[k] = all[k];
+    }
     if (ch.root) {
       T c = T(0);
 #pragma unroll
-      for (int k = 0; k < K; ++k) c += y[k];
+      for (int k = 0; k < K; ++k) c += all[k];
       c = sum_to_lane63(c);
       if (lane == 63) sc.add(0u, c);
     }

@@ -23,12 +23,24 @@ __global__ void tree_weights_kernel(const double* __restrict__ alpha,
   if (e < n) W[e] = ti[e] >= 0 ? static_cast<T>(alpha[ti[e]]) : T(0);
 }
 
+// a product in two doubles (one rounding in the end instead of one a factor)
+struct Product {
+  double hi = 1.0, lo = 0.0;
+  __device__ __forceinline__ void times(double f) {
+    const double p = hi * f;
+    lo = fma(hi, f, -p) + lo * f;
+    hi = p;
+  }
+  __device__ __forceinline__ double value() const { return hi + lo; }
+};
+
 // The data as the walks read them, in batches of 64 K rows (row 64 k + l of a
 // batch is lane l's point k): the lanes that multTranspose joins have consecutive
 // stored rows, and such groups are spread evenly over all rows. X: [D][ldx]. XT: per
-// dimension a row of 2^32 x; for Linear grids then per dimension a row of 2 over
-// the level-1 factor, and a row of the products of the level-1 factors. Rows past
-// M are copies of row M - 1 whose caller's row sperm is -1.
+// dimension a row of 2^32 x; for Linear grids then per dimension a row of 2^D times
+// the product of the later dimensions' halved level-1 factors (D <= kTreePassDims)
+// or of 2 over the level-1 factor, and a row of the products of the level-1 factors.
+// Rows past M are copies of row M - 1 whose caller's row sperm is -1.
 template <typename T, bool kMod>
 __global__ void tree_points_kernel(const T* __restrict__ X, int64_t ldx,
                                    const int32_t* __restrict__ dperm, int64_t M, int D, int K,
@@ -44,16 +56,23 @@ __global__ void tree_points_kernel(const T* __restrict__ X, int64_t ldx,
                     (lane % kGroup) * K + k;
   const int64_t from = m < M ? m : M - 1;
   sperm[r] = m < M ? dperm[m] : -1;
-  double all = 1.0;
-  for (int d = 0; d < D; ++d) {
+  const bool pass = D <= kTreePassDims;
+  Product all;
+  all.hi = ldexp(1.0, D);
+  for (int d = D - 1; d >= 0; --d) {
     const double x = static_cast<double>(X[d * ldx + from]);
     XT[d * rows + r] = static_cast<T>(x * 0x1.0p32);
     if (kMod) continue;
-    const double h = 2.0 * fmin(x, 1.0 - x);
-    XT[(D + d) * rows + r] = static_cast<T>(h < kTiny ? 0.0 : 2.0 / h);
-    all *= h < kTiny ? 0.0 : h;
+    double half = fmin(x, 1.0 - x);
+    if (pass) {
+      XT[(D + d) * rows + r] = static_cast<T>(all.value());
+    } else {
+      if (2.0 * half < kTiny) half = 0.0;
+      XT[(D + d) * rows + r] = static_cast<T>(half == 0.0 ? 0.0 : 1.0 / half);
+    }
+    all.times(half);
   }
-  if (!kMod) XT[2 * D * rows + r] = static_cast<T>(all);
+  if (!kMod) XT[2 * D * rows + r] = static_cast<T>(all.value());
 }
 
 // Y[r] = y[sperm[r]], 0 where sperm is -1
@@ -220,6 +239,7 @@ void append_program(const TreeGrid& g, size_t a, size_t b, int64_t off0, int ent
                        flags});
     path = steps;
   }
+  int passed[kTreeMaxDepth] = {};  // per depth: the dimensions before this one are passed
   for (size_t i = 0; i < out.size(); ++i) {
     Emit& e = out[i];
     if (i + 1 < out.size() && out[i + 1].depth == e.depth + 1) e.flags |= kTreePush;
@@ -235,6 +255,13 @@ void append_program(const TreeGrid& g, size_t a, size_t b, int64_t off0, int ent
             e.flags;
     r.scale = fp32 ? static_cast<uint32_t>(127 + e.level - 33) << 23
                    : static_cast<uint32_t>(1023 + e.level - 33) << 20;
+    if (g.D <= kTreePassDims) {
+      // from the parent's dimension, or the run before, to this record's
+      if (i == 0 || out[i - 1].depth < e.depth)
+        passed[e.depth] = e.depth > 0 ? out[i - 1].dim + 1 : 0;
+      r.ctl |= static_cast<uint32_t>(e.dim - passed[e.depth]) << kTreePassShift;
+      passed[e.depth] = e.dim;
+    }
     p.recs.push_back(r);
   }
 }
