@@ -428,13 +428,23 @@ struct TreeScatter {
   }
 };
 
+// Waves per SIMD: three where four (128 registers) spill the coordinates and
+// products of several points. Kernel times with four and three, level 5, 3e5
+// points: d=10 FP32 651 and 248 us, FP64 563 and 334; d=8 level 6, 5e5 points, FP32
+// 515 and 451; FP64 there spills two registers only, 579 and 648.
+template <typename T, int DB, int K, bool kMod>
+constexpr int tree_multT_waves() {
+  return kTreePass<DB, kMod> && K > 1 && DB >= (sizeof(T) == 4 ? 8 : 10) ? 3 : 4;
+}
+
 // Bound by vector instructions, the LDS adds about half of the time beside them.
 // Kernel times against the culled kernel: Linear d=8 level 6, 5e5 points, FP32
-// 1,621 to 515 us, FP64 2,300 to 579; ModLinear d=10 adaptive, 1e6 points, FP32
+// 1,621 to 451 us, FP64 2,300 to 579; ModLinear d=10 adaptive, 1e6 points, FP32
 // 2,218 to 1,903; against the subspace algorithm's own, d=7 level 6, 2.5e5 points,
 // 681 to 224 with the final sums.
 template <typename T, int DB, int K, bool kMod, int MD>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(tree_multT_waves<T, DB, K, kMod>())))
 void tree_multT_kernel(const TreeMultTArgs a) {
   const int lane = threadIdx.x;
   const TreeItem it = a.items[blockIdx.x];
