@@ -199,13 +199,14 @@ class DeviceMultiEval {
     int ngroups = 0;
     int lds = 0;  // bytes of the largest chunk's tables
   };
-  bool set_tree(const TreeGrid& g, bool mult, bool multT);
+  bool set_tree(const TreeGrid& g, const uint32_t* level, const uint32_t* index, bool mult,
+                bool multT);
   void release_tree();  // frees the walks' buffers
   // Kernels that evaluate a direction: the algorithm's own or the
   // subspace tree's
   enum class Path { Own, Tree };
-  bool set_paths(const TreeGrid* tree, const std::vector<double>& li,
-                 const std::vector<uint32_t>& pmask);
+  bool set_paths(const TreeGrid* tree, const uint32_t* level, const uint32_t* index,
+                 const std::vector<double>& li, const std::vector<uint32_t>& pmask);
   double culled_cost(const std::vector<double>& li, const std::vector<uint32_t>& pmask) const;
   template <typename T>
   void set_tree_plans(const TreeGrid& g, bool mult, bool multT);

@@ -372,10 +372,10 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   std::vector<double> li0, sc0;
   encode_grid(basis_, D_, N, level, index, li0, sc0);
   TreeGrid tg;
-  const bool tree = build_tree_grid(D_, N, level, index, true, tg);
+  const bool tree = build_tree_grid(D_, N, level, tg);
   const size_t Npad = ((N + kGridPad - 1) / kGridPad) * kGridPad;
   N_ = 0;  // (set when the grid is laid out whole)
-  if (set_paths(tree ? &tg : nullptr, li0, pmask)) {
+  if (set_paths(tree ? &tg : nullptr, level, index, li0, pmask)) {
     N_ = N;
     Npad_ = Npad;
     return;
@@ -482,7 +482,8 @@ constexpr int64_t kTreePartWalks = 4;
 
 // Chooses the kernels of each direction (Path) and lays the grid out for them;
 // false if a direction is left to those of the instance's algorithm.
-bool DeviceMultiEval::set_paths(const TreeGrid* tree, const std::vector<double>& li,
+bool DeviceMultiEval::set_paths(const TreeGrid* tree, const uint32_t* level,
+                                const uint32_t* index, const std::vector<double>& li,
                                 const std::vector<uint32_t>& pmask) {
   mult_path_ = multT_path_ = Path::Own;
   if (!tree) return false;
@@ -503,7 +504,7 @@ bool DeviceMultiEval::set_paths(const TreeGrid* tree, const std::vector<double>&
   }
   if (!mult && !multT) return false;
   try {
-    if (!set_tree(*tree, mult, multT)) return false;
+    if (!set_tree(*tree, level, index, mult, multT)) return false;
   } catch (const device_error&) {
     // no memory for the walks' copy of the data, tables and programs (up to
     // three times the data): the other kernels need none of it

@@ -39,7 +39,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
 #include <vector>
 
 #include "cull_device.hpp"
@@ -277,57 +276,67 @@ int64_t subspace_table_limit(size_t N) {
   return std::max<int64_t>(int64_t(1) << 26, 64 * static_cast<int64_t>(N));
 }
 
+namespace {
+void check_points(size_t D, size_t N, const uint32_t* level, const uint32_t* index) {
+  for (size_t e = 0; e < N * D; ++e)
+    if (level[e] < 1 || level[e] > 30 || (index[e] & 1u) == 0 || index[e] >= (1u << level[e]))
+      throw input_error("invalid grid point (level/index out of range for a no-boundary grid)");
+}
+}  // namespace
+
 SubspaceLayout build_subspace_layout(size_t D, size_t N, const uint32_t* level,
                                      const uint32_t* index) {
   if (D > static_cast<size_t>(kSubMaxD))
     throw input_error("the subspace algorithm supports dimensions up to 20");
-  // group the points by level vector; std::map orders level vectors
-  // lexicographically, dimension 0 first
-  std::map<std::vector<uint8_t>, std::vector<uint32_t>> groups;
-  std::vector<uint8_t> lv(D);
+  check_points(D, N, level, index);
+  // the points by level vector, dimension 0 first: five bits a level, 12 in a word
+  struct Key {
+    uint64_t w[2];
+    uint32_t j;
+  };
+  std::vector<Key> key(N);
   for (size_t j = 0; j < N; ++j) {
-    for (size_t d = 0; d < D; ++d) {
-      const uint32_t l = level[j * D + d], i = index[j * D + d];
-      if (l < 1 || l > 30 || (i & 1u) == 0 || i >= (1u << l))
-        throw input_error("invalid grid point (level/index out of range for a no-boundary grid)");
-      lv[d] = static_cast<uint8_t>(l);
-    }
-    groups[lv].push_back(static_cast<uint32_t>(j));
+    key[j] = Key{{0, 0}, static_cast<uint32_t>(j)};
+    for (size_t d = 0; d < D; ++d)
+      key[j].w[d / 12] |= static_cast<uint64_t>(level[j * D + d]) << (5 * (11 - d % 12));
   }
+  std::sort(key.begin(), key.end(), [](const Key& x, const Key& y) {
+    return x.w[0] != y.w[0] ? x.w[0] < y.w[0] : (x.w[1] != y.w[1] ? x.w[1] < y.w[1] : x.j < y.j);
+  });
   SubspaceLayout lay;
-  lay.desc.reserve(groups.size() + kSubBatch - 1);
   lay.te.resize(N);
-  const std::vector<uint8_t>* prev = nullptr;
-  for (const auto& g : groups) {
+  std::vector<size_t> first;  // per subspace its first point in key
+  const uint32_t* prev = nullptr;
+  for (size_t s = 0; s < N; ++s) {
+    if (s && key[s].w[0] == key[s - 1].w[0] && key[s].w[1] == key[s - 1].w[1]) continue;
+    const uint32_t* lv = level + static_cast<size_t>(key[s].j) * D;
     int levelsum = 0;
-    for (size_t d = 0; d < D; ++d) levelsum += g.first[d] - 1;
+    for (size_t d = 0; d < D; ++d) levelsum += static_cast<int>(lv[d]) - 1;
     if (levelsum > 30) throw input_error("a subspace's index table would exceed 2^30 entries");
     SubspaceDesc sd{};
     sd.off = lay.total;
-    int r = 0;
-    if (prev)
-      while (r < static_cast<int>(D) && (*prev)[r] == g.first[r]) ++r;
-    sd.recalc = prev ? r : 0;
-    for (size_t d = 0; d < D; ++d) sd.level[d] = g.first[d];
+    while (prev && prev[sd.recalc] == lv[sd.recalc]) ++sd.recalc;
+    for (size_t d = 0; d < D; ++d) sd.level[d] = static_cast<unsigned char>(lv[d]);
     lay.desc.push_back(sd);
     lay.total += int64_t(1) << levelsum;
-    prev = &g.first;
+    first.push_back(s);
+    prev = lv;
   }
+  first.push_back(N);
   // a table entry per cell of every subspace; refuse tables far larger than the grid
   if (lay.total > subspace_table_limit(N))
     throw input_error("the subspace index tables of this grid would hold more than 64 entries "
                       "per grid point");
   lay.ti.assign(static_cast<size_t>(lay.total), -1);
-  size_t s = 0;
-  for (const auto& g : groups) {
-    for (uint32_t j : g.second) {
+  for (size_t q = 0; q + 1 < first.size(); ++q)
+    for (size_t s = first[q]; s < first[q + 1]; ++s) {
+      const size_t j = key[s].j;
+      const SubspaceDesc& sd = lay.desc[q];
       int64_t flat = 0;
-      for (size_t d = 0; d < D; ++d) flat = (flat << (g.first[d] - 1)) + (index[j * D + d] >> 1);
-      lay.ti[static_cast<size_t>(lay.desc[s].off + flat)] = static_cast<int32_t>(j);
-      lay.te[j] = lay.desc[s].off + flat;
+      for (size_t d = 0; d < D; ++d) flat = (flat << (sd.level[d] - 1)) + (index[j * D + d] >> 1);
+      lay.ti[static_cast<size_t>(sd.off + flat)] = static_cast<int32_t>(j);
+      lay.te[j] = sd.off + flat;
     }
-    ++s;
-  }
   lay.nsub = static_cast<int>(lay.desc.size());
   lay.desc.resize(lay.desc.size() + kSubBatch - 1, SubspaceDesc{});  // batch padding
   return lay;
@@ -335,37 +344,39 @@ SubspaceLayout build_subspace_layout(size_t D, size_t N, const uint32_t* level,
 
 void DeviceMultiEval::set_grid_subspace(const uint32_t* level, const uint32_t* index, size_t N) {
   check_hip(hipSetDevice(device_), "hipSetDevice");
+  check_points(D_, N, level, index);
   TreeGrid tg;
-  build_tree_grid(D_, N, level, index, false, tg);
-  // the subspaces in lexicographic order: the dimensions evaluated per data row
-  // (those shared with the previous one left out), and the chunks of this
-  // algorithm's multTranspose
-  std::vector<const uint8_t*> lv(tg.node.size());
-  for (size_t s = 0; s < lv.size(); ++s) lv[s] = &tg.level[s * D_];
-  std::sort(lv.begin(), lv.end(), [&](const uint8_t* a, const uint8_t* b) {
-    return std::lexicographical_compare(a, a + D_, b, b + D_);
-  });
-  uint64_t steps = 0;
-  int64_t nchunk = 0, fill = kSubLds;
-  for (size_t s = 0; s < lv.size(); ++s) {
-    int bits = 0;
-    for (size_t d = 0; d < D_; ++d) bits += lv[s][d] - 1;
-    const int64_t n = int64_t(1) << bits;
-    if (fill + n > kSubLds) ++nchunk;
-    fill = n > kSubLds ? kSubLds : (fill + n > kSubLds ? n : fill + n);
-    size_t d = 0;
-    while (s && lv[s][d] == lv[s - 1][d]) ++d;
-    for (; d < D_; ++d) steps += !(basis_ == Basis::ModLinear && lv[s][d] == 1);
-  }
-  if (nchunk > 65535) throw input_error("too many subspace chunks for one launch");
-  N_ = 0;  // (set when the grid is laid out whole)
-  if (set_paths(&tg, {}, {})) {
-    N_ = N;
-    Npad_ = N;
-    nsub_ = static_cast<int>(tg.node.size());
-    ntable_ = tg.total;
-    sub_recompute_ = sub_recompute_t_ = steps;
-    return;
+  if (build_tree_grid(D_, N, level, tg)) {
+    // the subspaces in lexicographic order: the dimensions evaluated per data row
+    // (those shared with the previous one left out), and the chunks of this
+    // algorithm's multTranspose
+    std::vector<const uint8_t*> lv(tg.node.size());
+    for (size_t s = 0; s < lv.size(); ++s) lv[s] = &tg.level[s * D_];
+    std::sort(lv.begin(), lv.end(), [&](const uint8_t* a, const uint8_t* b) {
+      return std::lexicographical_compare(a, a + D_, b, b + D_);
+    });
+    uint64_t steps = 0;
+    int64_t nchunk = 0, fill = kSubLds;
+    for (size_t s = 0; s < lv.size(); ++s) {
+      int bits = 0;
+      for (size_t d = 0; d < D_; ++d) bits += lv[s][d] - 1;
+      const int64_t n = int64_t(1) << bits;
+      if (fill + n > kSubLds) ++nchunk;
+      fill = n > kSubLds ? kSubLds : (fill + n > kSubLds ? n : fill + n);
+      size_t d = 0;
+      while (s && lv[s][d] == lv[s - 1][d]) ++d;
+      for (; d < D_; ++d) steps += !(basis_ == Basis::ModLinear && lv[s][d] == 1);
+    }
+    if (nchunk > 65535) throw input_error("too many subspace chunks for one launch");
+    N_ = 0;  // (set when the grid is laid out whole)
+    if (set_paths(&tg, level, index, {}, {})) {
+      N_ = N;
+      Npad_ = N;
+      nsub_ = static_cast<int>(tg.node.size());
+      ntable_ = tg.total;
+      sub_recompute_ = sub_recompute_t_ = steps;
+      return;
+    }
   }
   SubspaceLayout lay = build_subspace_layout(D_, N, level, index);
   std::vector<SubspaceDesc>& desc = lay.desc;
@@ -386,6 +397,8 @@ void DeviceMultiEval::set_grid_subspace(const uint32_t* level, const uint32_t* i
     chunks.back().n += static_cast<int>(n);
   }
   if (chunks.size() > 65535) throw input_error("too many subspace chunks for one launch");
+  N_ = 0;
+  mult_path_ = multT_path_ = Path::Own;
   check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
   Npad_ = N;
   nchunk_ = static_cast<int>(chunks.size());

@@ -109,17 +109,19 @@ struct TreeGrid {
   size_t D = 0;
   std::vector<uint8_t> level;  // [nodes][D]
   std::vector<Node> node;
-  std::vector<int32_t> ti;     // grid point of a table entry, or -1
+  std::vector<uint32_t> order; // the grid points by node
+  std::vector<uint32_t> first; // per node its first in order, and their number
   int64_t total = 0;           // table entries
   int depth = 0;               // of the deepest node
-  bool repeated = false;       // a grid point occurs twice (a table holds it once)
 };
-// Sorts the points by subspace and builds the tables. Throws input_error
-// for points outside a no-boundary grid and for tables beyond
-// subspace_table_limit(N) or 2^30 cells in one subspace; with quiet it returns
-// false for the latter two instead.
-bool build_tree_grid(size_t D, size_t N, const uint32_t* level, const uint32_t* index,
-                     bool quiet, TreeGrid& g);
+// Sorts the points of a no-boundary grid by subspace. False for grids that the walks
+// do not cover: more than kTreeMaxDepth levels above 1 in a level vector, tables
+// beyond subspace_table_limit(N) or 2^30 cells in one subspace.
+bool build_tree_grid(size_t D, size_t N, const uint32_t* level, TreeGrid& g);
+// The grid point of every table entry, or -1; false if a grid point occurs twice
+// (a table holds it once).
+bool tree_tables(const TreeGrid& g, const uint32_t* level, const uint32_t* index,
+                 std::vector<int32_t>& ti);
 
 // Nodes to walk per data point, those of tables in parts counted per part (and
 // their ancestors).

@@ -5,8 +5,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <cstring>
-#include <numeric>
 
 #include "parts_device.hpp"
 #include "tree_device.hpp"
@@ -97,100 +95,93 @@ __global__ __launch_bounds__(kRows* kCols) void tree_sum_kernel(
 
 }  // namespace
 
-bool build_tree_grid(size_t D, size_t N, const uint32_t* level, const uint32_t* index,
-                     bool quiet, TreeGrid& g) {
-  g = TreeGrid();
-  g.D = D;
-  for (size_t e = 0; e < N * D; ++e) {
-    const uint32_t l = level[e], i = index[e];
-    if (l < 1 || l > 30 || (i & 1u) == 0 || i >= (1u << l))
-      throw input_error("invalid grid point (level/index out of range for a no-boundary grid)");
-  }
-  // points by subspace in depth-first order: the steps (dimension, level above
-  // 1) compare one by one, a parent before its children. As numbers per
-  // dimension: the level, or for level 1 a value above all levels where
-  // another step follows (its dimension is larger) and 0 where none does.
-  // 5 bits each: two words hold 24 dimensions.
-  std::vector<uint32_t> order(N);
-  std::iota(order.begin(), order.end(), 0u);
-  if (D <= 24) {
-    struct Key {
-      uint64_t a, b;
-      uint32_t j;
-    };
-    std::vector<Key> key(N);
-    for (size_t j = 0; j < N; ++j) {
-      uint64_t w[2] = {0, 0};
-      bool later = false;
-      for (size_t d = D; d-- > 0;) {
-        const uint64_t l = level[j * D + d];
-        w[d / 12] |= (l > 1 ? l : (later ? 31u : 0u)) << (5 * (11 - d % 12));
-        later |= l > 1;
+namespace {
+
+// The steps of a level vector, (dimension, level above 1) one by one: five of 12 bits
+// in a word, the first at the top, 0 where there is none. So keys compare as the
+// depth-first order does, a parent before its children.
+constexpr int kStepsPerWord = 5;
+template <int W>
+struct StepKey {
+  uint64_t w[W];
+  uint32_t j;
+  bool same(const StepKey& o) const { return std::equal(w, w + W, o.w); }
+};
+
+template <int W>
+bool tree_nodes(size_t D, size_t N, const uint32_t* level, TreeGrid& g) {
+  std::vector<StepKey<W>> key(N);
+  for (size_t j = 0; j < N; ++j) {
+    StepKey<W>& k = key[j];
+    k = StepKey<W>{};
+    k.j = static_cast<uint32_t>(j);
+    int n = 0;
+    for (size_t d = 0; d < D; ++d)
+      if (const uint64_t l = level[j * D + d]; l > 1) {
+        k.w[n / kStepsPerWord] |= ((d + 1) << 5 | l) << (12 * (kStepsPerWord - 1 - n % kStepsPerWord));
+        ++n;
       }
-      key[j] = Key{w[0], w[1], static_cast<uint32_t>(j)};
-    }
-    std::sort(key.begin(), key.end(), [](const Key& x, const Key& y) {
-      return x.a != y.a ? x.a < y.a : (x.b != y.b ? x.b < y.b : x.j < y.j);
-    });
-    for (size_t s = 0; s < N; ++s) order[s] = key[s].j;
-  } else {
-    auto later = [&](const uint32_t* p, size_t d) {
-      while (++d < D)
-        if (p[d] > 1) return true;
-      return false;
-    };
-    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
-      const uint32_t *p = level + x * D, *q = level + y * D;
-      for (size_t d = 0; d < D; ++d)
-        if (p[d] != q[d]) {
-          if (p[d] == 1) return !later(p, d);
-          if (q[d] == 1) return later(q, d);
-          return p[d] < q[d];
-        }
-      return x < y;
-    });
   }
+  std::sort(key.begin(), key.end(), [](const StepKey<W>& x, const StepKey<W>& y) {
+    for (int i = 0; i < W; ++i)
+      if (x.w[i] != y.w[i]) return x.w[i] < y.w[i];
+    return x.j < y.j;
+  });
   const int64_t limit = subspace_table_limit(N);
+  g.order.resize(N);
   for (size_t s = 0; s < N; ++s) {
-    const uint32_t* lv = level + static_cast<size_t>(order[s]) * D;
-    if (s && std::memcmp(level + static_cast<size_t>(order[s - 1]) * D, lv, D * sizeof(uint32_t)) == 0)
-      continue;
+    g.order[s] = key[s].j;
+    if (s && key[s].same(key[s - 1])) continue;
     TreeGrid::Node n{0, g.total, 0};
+    const uint32_t* lv = level + static_cast<size_t>(key[s].j) * D;
     int64_t bits = 0;
     for (size_t d = 0; d < D; ++d) {
       n.depth += lv[d] > 1;
       bits += lv[d] - 1;
       g.level.push_back(static_cast<uint8_t>(lv[d]));
     }
-    if (bits > 30) {
-      if (quiet) return false;
-      throw input_error("a subspace's index table would exceed 2^30 entries");
-    }
+    if (bits > 30) return false;
     n.bits = static_cast<int>(bits);
     g.total += int64_t(1) << bits;
-    if (g.total > limit) {
-      if (quiet) return false;
-      throw input_error("the subspace index tables of this grid would hold more than 64 entries "
-                        "per grid point");
-    }
-    g.depth = std::max(g.depth, n.depth);
+    if (g.total > limit) return false;
     g.node.push_back(n);
+    g.first.push_back(static_cast<uint32_t>(s));
   }
-  g.ti.assign(static_cast<size_t>(g.total), -1);
-  size_t at = 0;
-  for (size_t s = 0; s < N; ++s) {
-    const uint32_t* lv = level + static_cast<size_t>(order[s]) * D;
-    const uint32_t* ix = index + static_cast<size_t>(order[s]) * D;
-    if (s) {
-      const uint32_t* before = level + static_cast<size_t>(order[s - 1]) * D;
-      if (std::memcmp(before, lv, D * sizeof(uint32_t)) != 0) ++at;
+  g.first.push_back(static_cast<uint32_t>(N));
+  return true;
+}
+
+}  // namespace
+
+bool build_tree_grid(size_t D, size_t N, const uint32_t* level, TreeGrid& g) {
+  g = TreeGrid();
+  g.D = D;
+  for (size_t j = 0; j < N; ++j) {
+    int n = 0;
+    for (size_t d = 0; d < D; ++d) n += level[j * D + d] > 1;
+    g.depth = std::max(g.depth, n);
+  }
+  if (g.depth > kTreeMaxDepth) return false;
+  static_assert(kTreeMaxDepth <= 3 * kStepsPerWord, "a key holds every step");
+  if (g.depth <= kStepsPerWord) return tree_nodes<1>(D, N, level, g);
+  if (g.depth <= 2 * kStepsPerWord) return tree_nodes<2>(D, N, level, g);
+  return tree_nodes<3>(D, N, level, g);
+}
+
+bool tree_tables(const TreeGrid& g, const uint32_t* level, const uint32_t* index,
+                 std::vector<int32_t>& ti) {
+  ti.assign(static_cast<size_t>(g.total), -1);
+  for (size_t q = 0; q < g.node.size(); ++q)
+    for (uint32_t s = g.first[q]; s < g.first[q + 1]; ++s) {
+      const size_t j = g.order[s];
+      int64_t flat = 0;
+      for (size_t d = 0; d < g.D; ++d)
+        if (const uint32_t l = level[j * g.D + d]; l > 1)
+          flat = (flat << (l - 1)) + (index[j * g.D + d] >> 1);
+      int32_t& entry = ti[static_cast<size_t>(g.node[q].off + flat)];
+      if (entry >= 0) return false;
+      entry = static_cast<int32_t>(j);
     }
-    int64_t flat = 0;
-    for (size_t d = 0; d < D; ++d) flat = (flat << (lv[d] - 1)) + (ix[d] >> 1);
-    int32_t& entry = g.ti[static_cast<size_t>(g.node[at].off + flat)];
-    g.repeated |= entry >= 0;
-    entry = static_cast<int32_t>(order[s]);
-  }
   return true;
 }
 
@@ -481,12 +472,14 @@ int64_t tree_walks(const TreeGrid& g, bool multT) {
   return n;
 }
 
-bool DeviceMultiEval::set_tree(const TreeGrid& g, bool mult, bool multT) {
-  if (g.repeated || g.depth > kTreeMaxDepth || g.node.size() > (size_t(1) << 24)) return false;
+bool DeviceMultiEval::set_tree(const TreeGrid& g, const uint32_t* level, const uint32_t* index,
+                               bool mult, bool multT) {
+  std::vector<int32_t> ti;
+  if (g.node.size() > (size_t(1) << 24) || !tree_tables(g, level, index, ti)) return false;
   check_hip(hipSetDevice(device_), "hipSetDevice");
   check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-  ensure(&tree_ti_, &tree_ti_cap_, g.ti.size() * sizeof(int32_t));
-  check_hip(hipMemcpy(tree_ti_, g.ti.data(), g.ti.size() * sizeof(int32_t), hipMemcpyHostToDevice),
+  ensure(&tree_ti_, &tree_ti_cap_, ti.size() * sizeof(int32_t));
+  check_hip(hipMemcpy(tree_ti_, ti.data(), ti.size() * sizeof(int32_t), hipMemcpyHostToDevice),
             "upload tables");
   tree_total_ = g.total;
   tree_nodes_ = static_cast<int64_t>(g.node.size());

@@ -90,3 +90,29 @@ def test_no_memory_for_the_walks(on_host, algorithm, precision):
         print(own)
     """ % (precision, algorithm))
     assert int(out) >= 5
+
+
+def test_tables_only_for_walked_grids(on_host):
+    """A deep grid around one point: 144 points in 16.8 million cells of their subspaces. No
+    table of them is filled for a grid that keeps the culled kernels (67 MB), and no second one
+    for one that keeps the subspace kernels."""
+    out = on_host("""
+        import resource
+        l = np.arange(1, 13)
+        lv = np.ones((144, 3), np.uint32)
+        lv[:, 0], lv[:, 1] = np.repeat(l, 12), np.tile(l, 12)
+        ix = 2 * (0.3 * 2.0 ** (lv - 1.0)).astype(np.uint32) + 1
+        X = workloads.uniform_points(1, 500, 3)
+        peak = [resource.getrusage(resource.RUSAGE_SELF).ru_maxrss]
+        for algorithm in (0, 1):
+            op = capi.MultiEval(1, X, algorithm=algorithm).prepare(lv, ix)
+            peak.append(resource.getrusage(resource.RUSAGE_SELF).ru_maxrss)
+            launches()
+            op.mult(np.zeros(144))
+            assert not any("tree" in name for name, _, _, _ in launches())
+            op = None
+        print(peak[1] - peak[0], peak[2] - peak[1])
+    """)
+    streaming, subspace = (int(v) / 1024 for v in out.split())  # MiB
+    assert streaming < 32
+    assert subspace < 64 + 64 + 32  # the table, and the copy that stands for the GPU's
