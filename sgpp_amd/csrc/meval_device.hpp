@@ -207,7 +207,16 @@ class DeviceMultiEval {
   enum class Path { Own, Tree };
   bool set_paths(const TreeGrid* tree, const uint32_t* level, const uint32_t* index,
                  const std::vector<double>& li, const std::vector<uint32_t>& pmask);
+  // expected times of both directions, in us
+  struct PathTimes {
+    double mult, multT;
+  };
+  PathTimes tree_times(const TreeGrid& g) const;
+  PathTimes own_times(const TreeGrid& g, const std::vector<double>& li,
+                      const std::vector<uint32_t>& pmask) const;
   double culled_cost(const std::vector<double>& li, const std::vector<uint32_t>& pmask) const;
+  template <typename T>
+  bool tree_wide(const TreeGrid& g) const;
   template <typename T>
   void set_tree_plans(const TreeGrid& g, bool mult, bool multT);
   template <typename T>

@@ -448,60 +448,83 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
   }
 }
 
-// The subspace tree's walks cost the same per node and data point whatever the
-// data; the culled kernels' cost follows the grid points that a data group's box
-// meets, estimated on a few groups and grid points (two per evaluated dimension and
-// 2.5 more, per node). Culled against walked, mult and multTranspose in us:
-//   cost   7, d=10, 1,880 nodes, M=5e6, FP32   2,295 to 3,184   2,447 to 4,671
-//   cost  11, d=10, 3,418 nodes, M=5e6, FP32   7,185 to 6,049   7,493 to 8,730
-//   cost  15, d=10, 3,418 nodes, M=1e6, FP32   2,051 to 1,403   2,218 to 1,880
-//   cost  16, d=20, 14,650 nodes, M=5e6, FP32 38,185 to 29,890  30,118 to 47,319
-//   cost  24, d=20, 14,650 nodes, M=5e5, FP32  6,523 to 3,023   5,326 to 4,917
-//   cost   6, d=10, 9,212 nodes up to 7 dimensions refined, M=2e6, FP32
-//                                              3,355 to 14,501  3,623 to 20,853
-//   cost  12, the same with 1,223 nodes, d=8, FP64
-//                                              4,055 to 2,105   4,162 to 3,184
-//   cost 109, d=8, 1,287 nodes, M=5e5, FP32    1,179 to 246     1,621 to 469
-// Below kTreeSmallWork nodes times data points the culled kernels are bound by
-// their tests and launches and the walks won at every cost measured (8 and more).
-constexpr double kTreeSmallWork = 2e9;
-constexpr double kTreeCostSmall = 5.0;
-// the cost above which a walk is the faster ({mult, multTranspose}; walks of more
-// than kTreeFewDims refined dimensions take one data point per lane)
-struct TreeCosts {
-  double mult, multT;
-};
-TreeCosts tree_costs(bool fp32, bool wide_dims, bool deep) {
-  if (fp32) return deep ? TreeCosts{22.0, 30.0} : TreeCosts{11.0, wide_dims ? 22.0 : 13.5};
-  return deep ? TreeCosts{9.0, 12.0} : TreeCosts{7.0, 10.0};
-}
+// What the kernels of the instance's algorithm take, in us, to be held against
+// tree_times(). Fitted to 842 pairs of both (each basis, precision and algorithm; 1 to 60
+// dimensions, 41 to 100,000 grid points, 300 to 8e6 data points). The kernels
+// chosen by the fits take 1.2 % more than the faster ones of each pair.
+//
+// Culled: a cost per data point, the grid points that a data group's box meets (two
+// per evaluated dimension and 2.5 more), estimated on a few groups and grid points, and
+// a wave's share of it as a chain: a block's first group meets its chunk (256 grid
+// points of mult, kChunkT of multTranspose) with no other wave's work beside it,
+// three and four times as dense as on average. ModLinear points share dimensions
+// less the more there are.
+// Generic (no culling): every pair and dimension; chains as above.
+// Subspace: a thread's chain of all nodes, and the evaluated dimensions.
+//
+// Own against walked on either side of the lines, in us (grid points, data points):
+//   FP32 mult    ModLinear d=6  20,337, 5e6   1,170 1,393   Linear d=3   3,075, 8e6    486   412
+//                Linear d=13    22,026, 1e6   1,346 2,290   ModLinear d=13 20,863, 3e6 2,906 2,423
+//        multT   ModLinear d=10 100,015, 5e6  7,399 8,723   the same, 1e6              2,149 1,842
+//                Linear d=13    22,026, 2e5     708   822   ModLinear d=20 21,794, 2e5 1,164   958
+//   FP64 mult    Linear d=4      3,665, 1e6     163   194   Linear d=8   4,364, 2e5      199   166
+//                Linear d=13     5,981, 1e6     986 1,204   Linear d=13 22,026, 2e5    1,257   960
+//        multT   ModLinear d=10 21,165, 3e6   3,727 4,401   Linear d=5  20,362, 2e5      357   289
+//                Linear d=13     5,981, 1e6   1,299 1,980   the same, 2e5                530   452
+//   7 and 8 dimensions refined:
+//   FP32 mult    Linear d=8      1,530, 1e6     172   242   multT  ModLinear d=8 6,002, 1e6 460 375
+//   FP64 mult    ModLinear d=8   1,530, 1e6     167   244   multT  ModLinear d=8 6,002, 1e6 510 398
+//   d=23 and 24: FP32 mult 500 points, 3.0 million table entries, 1e5 615 1,970; 64 points,
+//                65,025 entries, 1e5 169 72
+//   Subspace, d=10, 1,000 points, 858,148 entries, 4e5: both products 2,597 9,774; with
+//                47,916 entries 1,539 984
 constexpr size_t kProbePoints = 2048;
-// A table larger than a block's LDS is walked in parts; beyond this many walks
-// per node the subspace algorithm keeps its own kernels.
-constexpr int64_t kTreePartWalks = 4;
+
+DeviceMultiEval::PathTimes DeviceMultiEval::own_times(const TreeGrid& g,
+                                                      const std::vector<double>& li,
+                                                      const std::vector<uint32_t>& pmask) const {
+  const bool fp32 = serves(Precision::FP32), mod = basis_ == Basis::ModLinear;
+  const double M = static_cast<double>(M_), D = static_cast<double>(D_);
+  if (algorithm_ == Algorithm::Subspace) {
+    const double nodes = static_cast<double>(g.node.size());
+    return {17.0 + 0.353 * nodes + 0.16e-6 * nodes * D * M,
+            49.0 + 4e-6 * nodes * M + 34e-6 * static_cast<double>(g.total) + 400e-6 * M};
+  }
+  const double N = static_cast<double>(pmask.size());
+  if (D_ > static_cast<size_t>(kMaxTemplD)) {
+    const double tiles = std::ceil(N / kTG) * kTG;
+    return {(fp32 ? 0.2e-6 : 0.35e-6) * tiles * D * M +
+                (fp32 ? 0.08 : 0.1) * std::min(tiles, 4.0 * kTG) * D,
+            360.0 + (fp32 ? 1.9e-6 : 2.4e-6) * N * D * M};
+  }
+  const int dim = static_cast<int>(D_);
+  const double group = 1024.0 * 64.0 * (fp32 ? mult_k_rt<float>(dim) : mult_k_rt<double>(dim));
+  const double more = mod ? std::max(1.0, D / 10.0) : 1.0;
+  double c = fp32 ? 0.037 : 0.095, ct = fp32 ? 0.041 : 0.11;  // 1e-6 us per point and cost
+  if (!mod && D_ > 10) {
+    c = fp32 ? 0.034 : 0.055;
+    ct = fp32 ? 0.028 : 0.085;
+  } else if (!mod) {
+    c = fp32 ? 0.028 : 0.045;
+    ct = fp32 ? 0.032 : 0.057;
+  }
+  const double cost = 1e-6 * more * culled_cost(li, pmask);
+  return {42.0 + c * cost * (M + 3.0 * group * std::min(1.0, 4.0 * kTG / N)) + 35e-6 * M,
+          45.0 + ct * cost * (M + 4.0 * group * std::min(1.0, kChunkT / N)) + 65e-6 * M};
+}
 
 // Chooses the kernels of each direction (Path) and lays the grid out for them;
-// false if a direction is left to those of the instance's algorithm.
+// false if a direction is left to those of the instance's algorithm. (The subspace
+// algorithm's both or none: its layout and the tree's hold the same tables.)
 bool DeviceMultiEval::set_paths(const TreeGrid* tree, const uint32_t* level,
                                 const uint32_t* index, const std::vector<double>& li,
                                 const std::vector<uint32_t>& pmask) {
   mult_path_ = multT_path_ = Path::Own;
   if (!tree) return false;
-  const int64_t nodes = static_cast<int64_t>(tree->node.size());
-  const int64_t wm = tree_walks(*tree, false), wt = tree_walks(*tree, true);
-  bool mult = true, multT = true;
-  if (algorithm_ == Algorithm::Subspace) {
-    mult = wm <= kTreePartWalks * nodes;
-    multT = wt <= kTreePartWalks * nodes;
-  } else if (D_ <= static_cast<size_t>(kMaxTemplD)) {
-    const double cost = culled_cost(li, pmask);
-    const bool large = static_cast<double>(nodes) * static_cast<double>(M_) > kTreeSmallWork;
-    const TreeCosts t = large ? tree_costs(serves(Precision::FP32), D_ > 10,
-                                           tree->depth > kTreeFewDims)
-                              : TreeCosts{kTreeCostSmall, kTreeCostSmall};
-    mult = cost > t.mult * static_cast<double>(wm);
-    multT = cost > t.multT * static_cast<double>(wt);
-  }
+  const PathTimes own = own_times(*tree, li, pmask), walk = tree_times(*tree);
+  bool mult = walk.mult < own.mult, multT = walk.multT < own.multT;
+  if (algorithm_ == Algorithm::Subspace)
+    mult = multT = walk.mult + walk.multT < own.mult + own.multT;
   if (!mult && !multT) return false;
   try {
     if (!set_tree(*tree, level, index, mult, multT)) return false;

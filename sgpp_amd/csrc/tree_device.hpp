@@ -32,7 +32,7 @@ namespace sgpp_hip {
 // deeper grids are left to the other kernels.
 constexpr int kTreeMaxDepth = 12;
 // of the usual walks
-constexpr int kTreeFewDims = 6;
+constexpr int tree_few_dims(size_t D) { return D <= 4 ? 4 : 6; }
 
 // threads of a mult block (four waves share one chunk's tables)
 constexpr int kTreeBlock = 256;

@@ -505,7 +505,7 @@ constexpr int tree_k(int DB) {
 template <typename T, bool kMod, int DB>
 TreeLaunch tree_variant(int depth, bool wide) {
   constexpr int K = tree_k<T>(DB == 0 ? 20 : DB);
-  constexpr int kFew = DB == 4 ? 4 : kTreeFewDims;  // register sets of the usual variants
+  constexpr int kFew = tree_few_dims(DB == 0 ? 64 : DB);  // register sets of the usual variants
   TreeLaunch l;
   if (depth > kFew) {
     l.mult = &launch_tree_mult<T, DB, 1, kMod, kTreeMaxDepth>;

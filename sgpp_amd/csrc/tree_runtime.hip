@@ -332,6 +332,16 @@ constexpr int64_t kTreePartialBudget = int64_t(2048) << 20;
 
 }  // namespace
 
+int64_t tree_walks(const TreeGrid& g, bool multT) {
+  const int64_t cap = multT ? kMultTEntries : kMultLds / 8;
+  int64_t n = 0;
+  for (const TreeGrid::Node& q : g.node) {
+    const int64_t size = int64_t(1) << q.bits;
+    n += size > cap ? (size + cap - 1) / cap * q.depth : 1;
+  }
+  return n;
+}
+
 void DeviceMultiEval::upload_tree(const TreeProgram& p, TreePlan& plan, int entry_bytes) {
   plan.ngroups = static_cast<int>(p.groups.size()) - 1;
   plan.lds = (p.max_entries * entry_bytes + 15) / 16 * 16;
@@ -349,21 +359,65 @@ void DeviceMultiEval::upload_tree(const TreeProgram& p, TreePlan& plan, int entr
             "upload tree groups");
 }
 
+namespace {
+
+template <typename T>
+TreeLaunch tree_variant_of(bool mod, size_t D, int depth, bool wide) {
+  return mod ? tree_launch<T, true>(static_cast<int>(D), depth, wide)
+             : tree_launch<T, false>(static_cast<int>(D), depth, wide);
+}
+
+// waves that the registers let a CU have in flight
+constexpr int64_t waves_per_cu(bool mod) { return mod ? 16 : 12; }
+
+}  // namespace
+
+// several points per lane where that leaves every wave slot a walk of kMinNodes
+template <typename T>
+bool DeviceMultiEval::tree_wide(const TreeGrid& g) const {
+  const bool mod = basis_ == Basis::ModLinear;
+  return static_cast<int64_t>(M_) * static_cast<int64_t>(g.node.size()) >=
+         num_cus_ * waves_per_cu(mod) * 64 * tree_variant_of<T>(mod, D_, g.depth, true).k * kMinNodes;
+}
+
+// The walks' times, fitted to the same pairs as own_times(): a launch or three; per
+// data point and node (parts of a table are walked each, with adds that meet in
+// multTranspose; walks of more than tree_few_dims() refined dimensions take one
+// point per lane, those of more than kRegDims dimensions read them from memory); what a block of mult
+// copies of the tables, and the chain of one table's parts; multTranspose's partial
+// sums and the rows that a final sum adds.
+DeviceMultiEval::PathTimes DeviceMultiEval::tree_times(const TreeGrid& g) const {
+  constexpr size_t kRegDims = 20;  // (of tree_launch)
+  // 1e-6 us per data point and node, mult and multTranspose: up to 10 dimensions,
+  // more, deep, more than kRegDims
+  constexpr double kNode[2][4][2] = {{{0.58, 1.11}, {0.77, 1.42}, {0.98, 1.54}, {1.3, 2.6}},
+                                     {{0.36, 0.67}, {0.42, 0.81}, {0.87, 1.35}, {0.9, 1.6}}};
+  const bool fp32 = serves(Precision::FP32), mod = basis_ == Basis::ModLinear;
+  const bool wide = fp32 ? tree_wide<float>(g) : tree_wide<double>(g);
+  const TreeLaunch l = fp32 ? tree_variant_of<float>(mod, D_, g.depth, wide)
+                            : tree_variant_of<double>(mod, D_, g.depth, wide);
+  const int c = D_ > kRegDims ? 3 : (g.depth > tree_few_dims(D_) ? 2 : (D_ > 10 ? 1 : 0));
+  const double M = static_cast<double>(M_), nodes = static_cast<double>(g.node.size()),
+               total = static_cast<double>(g.total),
+               walks = static_cast<double>(tree_walks(g, false)),
+               walksT = static_cast<double>(tree_walks(g, true));
+  const double blocks = std::ceil(M / (kTreeBlock * l.k));
+  const double rows = std::min(M / (64 * l.k), 24576.0 / std::max(1.0, total / kMultTEntries));
+  return {20.0 + 1e-6 * (kNode[fp32][c][0] * walks + 8.0) * M + 1.2e-6 * total * blocks +
+              50e-6 * total + 0.25 * (walks - nodes),
+          25.0 + 1e-6 * (kNode[fp32][c][1] * (2.0 * walksT - nodes) + 15.0) * M + 25e-6 * total +
+              0.015 * rows};
+}
+
 template <typename T>
 void DeviceMultiEval::set_tree_plans(const TreeGrid& g, bool mult, bool multT) {
   const int ix = sizeof(T) == sizeof(double) ? 0 : 1;
   const bool mod = basis_ == Basis::ModLinear;
   const int64_t nodes = static_cast<int64_t>(g.node.size());
   const int64_t M = static_cast<int64_t>(M_);
-  const int64_t slots = static_cast<int64_t>(num_cus_) * (mod ? 16 : 12);
-  auto launch = [&](bool wide) {
-    return mod ? tree_launch<T, true>(static_cast<int>(D_), g.depth, wide)
-               : tree_launch<T, false>(static_cast<int>(D_), g.depth, wide);
-  };
-  // several points per lane where that leaves every wave slot a walk of kMinNodes
-  TreeLaunch l = launch(true);
-  tree_wide_[ix] = M * nodes >= slots * 64 * l.k * kMinNodes;
-  l = launch(tree_wide_[ix]);
+  const int64_t slots = num_cus_ * waves_per_cu(mod);
+  tree_wide_[ix] = tree_wide<T>(g);
+  const TreeLaunch l = tree_variant_of<T>(mod, D_, g.depth, tree_wide_[ix]);
   // the data in the walks' order
   const int64_t rb = (M + kTreeBlock * l.k - 1) / (kTreeBlock * l.k);
   const int64_t rows = tree_rows_[ix] = rb * kTreeBlock * l.k;
@@ -460,16 +514,6 @@ void DeviceMultiEval::set_tree_multT(const TreeGrid& g, int64_t batches) {
   ensure(&pt.sums, &pt.sums_cap, sums.size() * sizeof(TreeSum));
   check_hip(hipMemcpy(pt.sums, sums.data(), sums.size() * sizeof(TreeSum), hipMemcpyHostToDevice),
             "upload tree sums");
-}
-
-int64_t tree_walks(const TreeGrid& g, bool multT) {
-  const int64_t cap = multT ? kMultTEntries : kMultLds / 8;
-  int64_t n = 0;
-  for (const TreeGrid::Node& q : g.node) {
-    const int64_t size = int64_t(1) << q.bits;
-    n += size > cap ? (size + cap - 1) / cap * q.depth : 1;
-  }
-  return n;
 }
 
 bool DeviceMultiEval::set_tree(const TreeGrid& g, const uint32_t* level, const uint32_t* index,
