@@ -597,6 +597,7 @@ void DeviceMultiEval::choose_mult_order(const T* X, const T* LI, const float* TB
     // one; multTranspose runs on y = dR (zero: set above, and mult's output
     // on zero weights) and writes dA
     for (int kern = 0; kern < 2; ++kern) {
+      if ((kern == 0 ? mult_path_ : multT_path_) != Path::Own) continue;
       int& cf = kern == 0 ? mult_cf_[ix] : multT_cf_[ix];
       auto timed = [&]() {
         if (kern == 0)

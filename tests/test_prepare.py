@@ -1,7 +1,10 @@
 """Preparing a grid, on host memory: what a failed call leaves, and what a grid's layout takes."""
+import textwrap
+
 import pytest
 
 from host_hip import on_host  # noqa: F401
+from test_routes import GRIDS
 
 
 @pytest.mark.parametrize("algorithm", [0, 1])
@@ -116,3 +119,24 @@ def test_tables_only_for_walked_grids(on_host):
     streaming, subspace = (int(v) / 1024 for v in out.split())  # MiB
     assert streaming < 32
     assert subspace < 64 + 64 + 32  # the table, and the copy that stands for the GPU's
+
+
+@pytest.mark.parametrize("data,grid,culled", [
+    ("mixture(200000, 8)", "adaptive(8, 20000)", {"", "T"}),
+    ("uniform(200000, 1)", "regular(1, 10)", {"T"}),
+    ("uniform(10000, 5)", "regular(5, 5)", set())])
+def test_only_culled_directions_are_probed(on_host, data, grid, culled):
+    """The block order's timing launches are for the kernels that will run."""
+    on_host(GRIDS + textwrap.dedent("""
+        import re
+        X, (lv, ix) = %s, %s
+        op = capi.MultiEval(0, X, precision=1)
+        launches()
+        op.prepare(lv, ix)
+        probed = {m[1] for name, _, _, _ in launches() for m in [re.search("[0-9]mult(T?)_kernel", name)] if m}
+        assert probed == %r, probed
+        op.mult(np.zeros(op.N))
+        op.mult_transpose(np.zeros(op.M))
+        used = {m[1] for name, _, _, _ in launches() for m in [re.search("[0-9]mult(T?)_kernel", name)] if m}
+        assert used == probed, used
+    """) % (data, grid, culled))
