@@ -259,7 +259,8 @@ struct TreeWalk {
 
 extern __shared__ __align__(16) unsigned char tree_lds[];
 
-// byte address in LDS (the kernels have no LDS but tree_lds, which begins at 0)
+// byte address in LDS (the kernels have no LDS but tree_lds, which begins at 0: their
+// fixed size is tested. Adding tree_lds's address left an addition of 0 at every read)
 template <typename T>
 __device__ __forceinline__ T lds_read(unsigned a) {
   typedef const __attribute__((address_space(3))) T* Ptr;
@@ -451,6 +452,7 @@ void tree_multT_kernel(const TreeMultTArgs a) {
   const TreeChunk ch = a.chunks[it.chunk];
   double* acc = reinterpret_cast<double*>(tree_lds);
   for (int i = lane; i < ch.n; i += 64) acc[i] = 0.0;
+  __syncthreads();  // (one wave, whose LDS operations are in order: for the compiler)
   TreeScatter<T, K> sc;
   sc.part0 = ch.part0;
   sc.partn = ch.n;
@@ -479,7 +481,7 @@ void tree_multT_kernel(const TreeMultTArgs a) {
       walk.run((TreeRecPtr)(a.recs + ch.rec0), y);
     }
   }
-  // (one wave: its LDS operations are in order)
+  __syncthreads();
   double* out = a.part + it.off;
   for (int i = lane; i < ch.n; i += 64) out[i] = acc[i];
 }

@@ -54,3 +54,10 @@ def test_walks_keep_their_registers(kernels):
     assert len(walks) >= 64
     for v, *which in walks:
         assert int(v["private_segment_fixed_size"]) <= 48, which
+
+
+def test_walks_have_no_fixed_lds(kernels):
+    """The walks read LDS at byte offsets from address 0, where their dynamic LDS begins as long
+    as they declare no other."""
+    for v, *which in tree_kernels(kernels):
+        assert int(v["group_segment_fixed_size"]) == 0, which
