@@ -98,9 +98,9 @@ typedef struct sgpp_hip_params {
   int precision;        /* SGPP_HIP_PREC_* used by mult / mult_transpose */
   int keep_fp64;        /* also hold FP64 data when precision is FP32 */
   int device;           /* HIP device ordinal */
-  int mult_grid_chunks; /* 0 = automatic */
+  int mult_grid_chunks; /* 0 = automatic; walked grids: groups of subspaces */
   int multT_data_segs;  /* 0 = automatic */
-  int target_blocks;    /* 0 = automatic */
+  int target_blocks;    /* 0 = automatic; workgroups of a launch where neither is set */
   int algorithm;        /* SGPP_HIP_ALGO_* (0 = streaming) */
 } sgpp_hip_params;
 

@@ -441,11 +441,13 @@ void DeviceMultiEval::set_tree_mult(const TreeGrid& g, int64_t rb, int64_t slots
   TreePlan& pm = tree_mult_[sizeof(T) == sizeof(double) ? 0 : 1];
   const int64_t nodes = static_cast<int64_t>(g.node.size());
   const int64_t bslots = slots / (kTreeBlock / 64);
+  const int64_t gmax = std::max<int64_t>(1, nodes / kMinNodes);
   int64_t G = cfg_.mult_grid_chunks;
-  if (G <= 0) {
-    const int64_t gmax = std::max<int64_t>(1, std::min<int64_t>(64, nodes / kMinNodes));
+  if (G <= 0 && cfg_.target_blocks > 0) {
+    G = std::min(gmax, (cfg_.target_blocks + rb - 1) / rb);
+  } else if (G <= 0) {
     double best = 0.0;
-    for (int64_t q = 1; q <= gmax; ++q) {
+    for (int64_t q = 1; q <= std::min<int64_t>(64, gmax); ++q) {
       // nanoseconds per data point: the walk with the last round's idle
       // blocks, the FP64 partials written and read
       const double b = static_cast<double>(rb * q);
@@ -457,9 +459,10 @@ void DeviceMultiEval::set_tree_mult(const TreeGrid& g, int64_t rb, int64_t slots
         G = q;
       }
     }
-    G = std::min<int64_t>(G, std::max<int64_t>(1, kTreePartialBudget / (Mpad_ * sizeof(double))));
   }
-  upload_tree(build_tree_program(g, static_cast<int>(std::min<int64_t>(G, nodes)),
+  // (also where the caller sets G: the subspace algorithm's own kernels had no partials)
+  G = std::min<int64_t>(G, std::max<int64_t>(1, kTreePartialBudget / (Mpad_ * sizeof(double))));
+  upload_tree(build_tree_program(g, static_cast<int>(std::min<int64_t>({G, nodes, 65535})),
                                  (kMultLds - 16) / static_cast<int64_t>(sizeof(T)), nodes,
                                  static_cast<int>(sizeof(T)), sizeof(T) == 4),
               pm, static_cast<int>(sizeof(T)));
@@ -490,9 +493,9 @@ void DeviceMultiEval::set_tree_multT(const TreeGrid& g, int64_t batches) {
   pt.segs = 1;
   for (size_t c = 0; c < p.chunks.size(); ++c) {
     const TreeChunk& ch = p.chunks[c];
-    int64_t S = cfg_.multT_data_segs;
-    if (S <= 0)
-      S = static_cast<int64_t>(std::min(budget, target * (ch.nrec + kBatchNodes) / work + 0.5));
+    const double asked = cfg_.multT_data_segs > 0 ? cfg_.multT_data_segs
+                                                  : target * (ch.nrec + kBatchNodes) / work + 0.5;
+    int64_t S = static_cast<int64_t>(std::min(budget, asked));
     S = std::max<int64_t>(1, std::min<int64_t>(S, batches));
     const int64_t len = (batches + S - 1) / S;
     S = (batches + len - 1) / len;

@@ -70,3 +70,33 @@ def route(X, grid, basis, precision, algorithm):
 def test_routes(on_host, data, grid, basis, prec, algorithm, walked):
     out = on_host(GRIDS + "\nfor n in route(%s, %s, %d, %d, %d): print(n)" % (data, grid, basis, prec, algorithm))
     assert ["tree_mult" in line for line in out.splitlines()] == [walked == "both"] * 2, out
+
+
+def test_launch_knobs_of_walks(on_host):
+    """target_blocks sets the workgroups of both directions; chunks and segments that a caller
+    asks for stay within the partial sums' 2 GiB."""
+    on_host(GRIDS + """
+lv, ix = regular(6, 6)  # 462 subspaces
+X = uniform(100000, 6)
+
+def grids(**more):
+    op = capi.MultiEval(0, X, **more).prepare(lv, ix)
+    out = {}
+    for call, n in ((op.mult, op.N), (op.mult_transpose, op.M)):
+        launches()
+        hip.host_hip_clear()
+        call(np.zeros(n))
+        out["allocated"] = out.get("allocated", 0) + hip.host_hip_allocated()
+        for name, x, y, _ in launches():
+            if "tree_mult_k" in name: out["mult"] = x * y
+            if "tree_multT_k" in name: out["multT"] = x * y
+    return out
+
+few, many = grids(target_blocks=200), grids(target_blocks=4000)
+assert 200 <= few["mult"] <= 400 and 100 <= few["multT"] <= 400, few
+assert 4000 <= many["mult"] <= 4400 and 3000 <= many["multT"] <= 5000, many
+X = uniform(1500000, 6)
+for algorithm in (0, 1):
+    most = grids(mult_grid_chunks=1000000, multT_data_segs=1000000, algorithm=algorithm)
+    assert most["allocated"] <= 2 * (2048 << 20) + (64 << 20), most
+""")
