@@ -11,9 +11,9 @@ over all M x N pairs, with inputs resident in HBM.
 `value` is the FP32-with-FP64-accumulation form's pair-evals/s (2*M*N per
 step); the plain FP64 kernel is timed beside it ("fp64", "speedup_vs_fp64").
 Both forms' relative errors against the oracle are reported on a sample.
-roofline: the dominant FP32 kernel's executed flops (counted in the run by
-the counting instantiation of the same kernel) over its HIP-event time,
-against the FP32 vector peak; the 6d-per-pair figure over all M*N pairs is
+roofline: the dominant FP32 kernel's executed flops (of a culled kernel counted
+in the run by its counting instantiation, of a walk along the grid's subspaces its
+factors and look-ups for every data row) over its HIP-event time, against the FP32 vector peak; the 6d-per-pair figure over all M*N pairs is
 reported beside it as achieved_6d_convention.
 cpu_baseline: the reference's StreamingDefault ModLinear operator
 (OperationMultiEvalModMaskStreaming, compiled from the reference sources into
@@ -465,7 +465,8 @@ def solve_bench(args):
     sop = capi.MultiEval(capi.BASIS_LINEAR, X, algorithm=capi.ALGO_SUBSPACE).prepare(lv, ix)
     step_s, mult_ms, multT_ms = timed_steps(sop, capi.PREC_FP64, d_a, d_y, d_r, d_b, 5, 1, torch)
     kern["subspace_fp64"] = {"pair_evals_per_s": 2.0 * M * N / step_s, "mult_ms": mult_ms,
-                             "multT_ms": multT_ms, "executed_work": sop.count_work(capi.PREC_FP64)}
+                             "multT_ms": multT_ms, "kernels": sop.kernels(),
+                             "executed_work": sop.count_work(capi.PREC_FP64)}
     alpha_s, info_s = sop.solve(y, lam, max_iterations=10000, epsilon=1e-10, mode=capi.SOLVE_FP64)
     if ref is not None:
         info_s["alpha_rel_err_vs_cpu_fp64"] = float(np.linalg.norm(alpha_s - ref["alpha"]) /
@@ -566,11 +567,11 @@ def large_bench(args):
     launches = nm + nt
     flop_launch = 6.0 * d * M * N
     kern_s = (msm + mst) * 1e-3
-    dominant = "multT_kernel" if mst / nt >= msm / nm else "mult_kernel"
+    key = "multT" if mst / nt >= msm / nm else "mult"
+    dominant = op.kernels()[key == "multT"]
     dom_ms = max(mst / nt, msm / nm)
-    # executed work of one launch of each kernel (counting instantiations, untimed)
+    # executed work of one launch of each kernel (untimed)
     work = op.count_work(capi.PREC_FP32)
-    key = "multT" if dominant == "multT_kernel" else "mult"
     executed = 4.0 * work["%s_hat_steps" % key] + 2.0 * work["%s_pairs" % key]
     note("CG done; subsample check")
     # subsample check: FP32 vs FP64 GPU products, FP64 vs the oracle
@@ -610,12 +611,8 @@ def large_bench(args):
                      "achieved_6d_convention": flop_launch / (dom_ms * 1e-3) / 1e12,
                      "flops_per_launch_6d_convention": flop_launch,
                      "traffic": None,
-                     "flop_convention": "achieved/frac: flops the kernel executes (4 per hat "
-                                        "step of an evaluated pair and dimension, 2 per "
-                                        "evaluated pair), counted by the counting "
-                                        "instantiation of the same kernel; "
-                                        "achieved_6d_convention: 6*d flops for every one of "
-                                        "the M*N pairs"},
+                     "flop_convention": flop_convention(dominant)},
+        "kernels": op.kernels(),
         "executed_work": work,
         "subsample": {
             "points": S,
@@ -691,7 +688,7 @@ def main():
         res[name] = dict(step_s=step_s, mult_ms=mult_ms, multT_ms=multT_ms,
                          shape=op.last_shape())
         outs[name] = (d_r.cpu().numpy().copy(), d_a.cpu().numpy().copy())
-    # executed work of each kernel (counting instantiations, untimed)
+    # executed work of each kernel (untimed)
     work = {name: op.count_work(prec) for name, prec in (("fp64", capi.PREC_FP64),
                                                           ("fp32", capi.PREC_FP32))}
 
@@ -702,8 +699,8 @@ def main():
 
     def roof(name, peak):
         k = res[name]
-        dom = "mult_kernel" if k["mult_ms"] >= k["multT_ms"] else "multT_kernel"
-        key = "mult" if dom == "mult_kernel" else "multT"
+        key = "mult" if k["mult_ms"] >= k["multT_ms"] else "multT"
+        dom = op.kernels()[key == "multT"]
         dom_ms = k["%s_ms" % key]
         w = work[name]
         executed = 4.0 * w["%s_hat_steps" % key] + 2.0 * w["%s_pairs" % key]
@@ -745,17 +742,11 @@ def main():
                  "roofline": dict(r64, bound="valu", kernel=dom64, unit="TFLOP/s")},
         "speedup_vs_fp64": v32 / v64,
         "kernel_ms_fp32": {"mult": k32["mult_ms"], "multT": k32["multT_ms"]},
+        "kernels": op.kernels(),
         "executed_work": work,
         "roofline": dict(r32, bound="valu", kernel=dom, unit="TFLOP/s", traffic=traffic,
                          traffic_source=tinfo,
-                         flop_convention="achieved/frac: flops the kernel executes, counted in "
-                                         "this run by the counting instantiation of the same "
-                                         "kernel (4 per hat step of an evaluated pair and "
-                                         "dimension, 2 per evaluated pair), over the kernel's "
-                                         "HIP-event time; achieved_6d_convention: 6*d flops for "
-                                         "every one of the M*N pairs "
-                                         "(LearnerVectorizedPerformanceCalculator), most of which "
-                                         "support culling skips as exact zeros"),
+                         flop_convention=flop_convention(dom)),
         "setup_s": setup_s,
     }
     # the subspace-indexed operator (FP64) on the same workload
@@ -766,6 +757,7 @@ def main():
     line["subspace_fp64"] = {
         "value": 2.0 * pairs / sstep, "unit": "pair-evals/s", "ms_per_step": sstep * 1e3,
         "mult_ms": smult, "multT_ms": smultT, "speedup_vs_streaming_fp64": res["fp64"]["step_s"] / sstep,
+        "kernels": sop.kernels(),
         "executed_work": sop.count_work(capi.PREC_FP64),
         "rel_diff_vs_streaming_fp64": {
             "mult": float(np.linalg.norm(rs - outs["fp64"][0]) / np.linalg.norm(outs["fp64"][0])),
@@ -784,6 +776,18 @@ def main():
     print(json.dumps(line))
 
 
+def flop_convention(kernel):
+    """what the roofline's flops count"""
+    how = ("4 per factor of the walk over the grid's subspaces and 2 per table look-up, for every "
+           "data row" if kernel.startswith("tree") else
+           "counted in this run by the counting instantiation of the same kernel: 4 per hat step of "
+           "an evaluated pair and dimension, 2 per evaluated pair")
+    return ("achieved/frac: flops the kernel executes (%s), over the kernel's HIP-event time; "
+            "achieved_6d_convention: 6*d flops for every one of the M*N pairs "
+            "(LearnerVectorizedPerformanceCalculator), most of which are exact zeros and are not "
+            "evaluated" % how)
+
+
 def profile_traffic(kernel, dtype):
     """HBM bytes per launch of the kernel from the committed rocprofv3 counter
     passes (profiles/traffic_<kernel>.json), used only when the profile was
@@ -791,7 +795,7 @@ def profile_traffic(kernel, dtype):
     import hashlib
     path = os.path.join(ROOT, "profiles", "traffic_%s.json" % kernel)
     h = hashlib.sha256()
-    for f in KERNEL_SOURCES:
+    for f in TREE_SOURCES if kernel.startswith("tree") else KERNEL_SOURCES:
         with open(os.path.join(ROOT, "sgpp_amd", "csrc", f), "rb") as fh:
             h.update(fh.read())
     digest = h.hexdigest()
@@ -807,6 +811,7 @@ def profile_traffic(kernel, dtype):
 
 
 KERNEL_SOURCES = ("meval_kernels.hpp", "cull_device.hpp", "meval_kernels.hip")
+TREE_SOURCES = ("tree_kernels.hpp", "cull_device.hpp", "tree_device.hpp", "tree_runtime.hip")
 
 
 if __name__ == "__main__":

@@ -104,7 +104,10 @@ typedef struct sgpp_hip_params {
   int algorithm;        /* SGPP_HIP_ALGO_* (0 = streaming) */
 } sgpp_hip_params;
 
-/* STREAMING: every (data point, grid point) pair, culled by supports
+/* The semantics of the operator; grids whose subspaces' index tables are small
+ * are evaluated subspace by subspace along a tree of their level vectors in
+ * either case, per direction where that is expected to be faster.
+ * STREAMING: every (data point, grid point) pair, culled by supports
  *   (OperationMultiEvalStreaming / OperationMultiEvalModMaskStreaming);
  * SUBSPACE: per data point and subspace the one basis function whose support
  *   holds the point, looked up in a dense per-subspace index table
@@ -180,12 +183,22 @@ sgpp_hip_status sgpp_hip_meval_last_shape(const sgpp_hip_meval* h, int* mult_chu
 sgpp_hip_status sgpp_hip_meval_kernel_timing_enable(sgpp_hip_meval* h, int on);
 sgpp_hip_status sgpp_hip_meval_kernel_timing(sgpp_hip_meval* h, int* n_mult, double* ms_mult,
                                              int* n_multT, double* ms_multT);
-/* Executed work of one mult and one multTranspose in the given precision,
- * counted by counting instantiations of the same kernels (launched untimed,
- * on zero inputs; culling does not depend on the values). out[0], out[1]:
- * mult hat steps (data point x grid point x evaluated dimension) and pairs
- * (every lane of every evaluated group of grid points); out[2], out[3]: the
- * same for multTranspose. No reference counterpart: the reference's operators
+/* The main kernels of the prepared grid's products, by name: the subspace
+ * tree's walks (tree_mult_kernel, tree_multT_kernel) or the algorithm's own
+ * (mult_kernel, mult_kernel_generic above 20 dimensions, subspace_mult_kernel,
+ * and the same with multT). */
+sgpp_hip_status sgpp_hip_meval_kernels(const sgpp_hip_meval* h, const char** mult,
+                                       const char** multT);
+/* Executed work of one mult and one multTranspose in the given precision.
+ * out[0], out[1]: mult hat steps (data point x grid point x evaluated
+ * dimension) and pairs; out[2], out[3]: the same for multTranspose. Culled
+ * kernels: counted by counting instantiations of the same kernels (launched
+ * untimed, on zero inputs; culling does not depend on the values), pairs in
+ * every lane of every evaluated group of grid points. Walks: data rows x the
+ * walk's factors, and x its table look-ups. SUBSPACE operators, whichever
+ * kernels run: the algorithm's count, data rows x subspaces (pairs) and x the
+ * dimensions that a subspace does not share with its predecessor (hat steps).
+ * No reference counterpart: the reference's operators
  * evaluate every pair, so LearnerVectorizedPerformanceCalculator
  * (datadriven/src/sgpp/datadriven/tools/LearnerVectorizedPerformanceCalculator.cpp:89-94)
  * counts all M x N pairs. */

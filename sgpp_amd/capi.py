@@ -165,6 +165,8 @@ SIGNATURES = {
                                         ctypes.POINTER(ctypes.c_int)]),
     "sgpp_hip_meval_kernel_timing_enable": (_st, [_p, ctypes.c_int]),
     "sgpp_hip_meval_mult_device_noalloc": (_st, [_p, _p, _p, ctypes.c_int]),
+    "sgpp_hip_meval_kernels": (_st, [_p, ctypes.POINTER(ctypes.c_char_p),
+                                     ctypes.POINTER(ctypes.c_char_p)]),
     "sgpp_hip_meval_count_work": (_st, [_p, ctypes.c_int, ctypes.POINTER(ctypes.c_uint64)]),
     "sgpp_hip_meval_kernel_timing": (_st, [_p, ctypes.POINTER(ctypes.c_int), _dp,
                                            ctypes.POINTER(ctypes.c_int), _dp]),
@@ -338,9 +340,10 @@ class Grid:
 class MultiEval:
     """OperationMultipleEval on the GPU (mult = B alpha, multTranspose = B^T y).
 
-    algorithm=ALGO_STREAMING: the culled streaming kernels (FP64 or FP32 with
-    FP64 accumulation); ALGO_SUBSPACE: the subspace-indexed kernels
-    (SubspaceLinear semantics, FP64, d <= 20)."""
+    algorithm=ALGO_STREAMING: streaming semantics (FP64 or FP32 with FP64
+    accumulation); ALGO_SUBSPACE: SubspaceLinear semantics (FP64, d <= 20).
+    Either walks the tree of the grid's subspaces, per direction, where that
+    is expected to be faster than its own kernels (kernels())."""
 
     def __init__(self, basis, data, precision=PREC_FP64, keep_fp64=False, device=0,
                  mult_grid_chunks=0, multT_data_segs=0, target_blocks=0, grid=None,
@@ -452,6 +455,12 @@ class MultiEval:
         check(F["sgpp_hip_meval_kernel_timing"](self.h, ctypes.byref(a), ctypes.byref(b),
                                                 ctypes.byref(c), ctypes.byref(d)))
         return a.value, b.value, c.value, d.value
+
+    def kernels(self):
+        """names of the main kernels of (mult, multTranspose) on the prepared grid"""
+        m, t = ctypes.c_char_p(), ctypes.c_char_p()
+        check(F["sgpp_hip_meval_kernels"](self.h, ctypes.byref(m), ctypes.byref(t)))
+        return m.value.decode(), t.value.decode()
 
     def count_work(self, precision):
         """Executed work of one mult and one multTranspose (counting kernels):

@@ -516,6 +516,16 @@ sgpp_hip_status sgpp_hip_meval_kernel_timing(sgpp_hip_meval* h, int* n_mult, dou
   });
 }
 
+sgpp_hip_status sgpp_hip_meval_kernels(const sgpp_hip_meval* h, const char** mult,
+                                       const char** multT) {
+  return guarded([&] {
+    REQUIRE(h && mult && multT, "null argument");
+    *mult = h->dev->kernel_name(false);
+    *multT = h->dev->kernel_name(true);
+    return SGPP_HIP_OK;
+  });
+}
+
 sgpp_hip_status sgpp_hip_meval_count_work(sgpp_hip_meval* h, int precision, uint64_t* out4) {
   return guarded([&] {
     REQUIRE(h && out4, "null argument");

@@ -127,6 +127,8 @@ class DeviceMultiEval {
   // subspace algorithm: number of subspaces and of index table entries
   int num_subspaces() const { return nsub_; }
   int64_t num_table_entries() const { return ntable_; }
+  // the main kernel of a direction for the prepared grid
+  const char* kernel_name(bool multT) const;
   bool serves(Precision p) const { return (precisions_ >> static_cast<int>(p)) & 1u; }
 
   // Kernel-only milliseconds of the last mult / multTranspose (HIP events).
@@ -198,6 +200,7 @@ class DeviceMultiEval {
     int nitems = 0, nsums = 0, segs = 0;
     int ngroups = 0;
     int lds = 0;  // bytes of the largest chunk's tables
+    int64_t factors = 0, lookups = 0;  // per data row: records, those with a table and the root
   };
   bool set_tree(const TreeGrid& g, const uint32_t* level, const uint32_t* index, bool mult,
                 bool multT);
@@ -286,7 +289,7 @@ class DeviceMultiEval {
   Path mult_path_ = Path::Own, multT_path_ = Path::Own;
   // subspace tree: its tables (grid point per entry, -1 where none), and per
   // precision (index 0 FP64, 1 FP32) the programs of mult and multTranspose
-  int64_t tree_total_ = 0, tree_nodes_ = 0;
+  int64_t tree_total_ = 0;
   int tree_depth_ = 0;
   void* tree_ti_ = nullptr;  size_t tree_ti_cap_ = 0;
   TreePlan tree_mult_[2], tree_multT_[2];

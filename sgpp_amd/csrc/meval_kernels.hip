@@ -874,20 +874,23 @@ void DeviceMultiEval::count_work(Precision p, uint64_t out[4]) {
   if (N_ == 0) throw input_error("grid not set (call prepare)");
   if (!serves(p)) throw input_error("precision not enabled for this instance");
   if (algorithm_ == Algorithm::Subspace) {
-    // every data row (padding included) visits every subspace and evaluates
-    // the dimensions it does not share with the previous one
+    // the algorithm's work, whichever kernels run: every data row (padding
+    // included) visits every subspace and evaluates the dimensions it does not
+    // share with the previous one
     out[1] = out[3] = static_cast<uint64_t>(Mpad_) * static_cast<uint64_t>(nsub_);
     out[0] = static_cast<uint64_t>(Mpad_) * sub_recompute_;
     out[2] = static_cast<uint64_t>(Mpad_) * sub_recompute_t_;
     return;
   }
-  // the tree: one factor and one pair per data row and node
-  const uint64_t walked = static_cast<uint64_t>(M_) * static_cast<uint64_t>(tree_nodes_);
-  if (mult_path_ != Path::Own && multT_path_ != Path::Own) {
-    out[0] = out[1] = walked;
-    out[2] = out[3] = walked;
-    return;
-  }
+  // a walk: every data row (padding included) takes the same records
+  const int ix = p == Precision::FP64 ? 0 : 1;
+  auto walked = [&](const TreePlan& plan, uint64_t* o) {
+    o[0] = static_cast<uint64_t>(tree_rows_[ix] * plan.factors);
+    o[1] = static_cast<uint64_t>(tree_rows_[ix] * plan.lookups);
+  };
+  if (mult_path_ != Path::Own) walked(tree_mult_[ix], out);
+  if (multT_path_ != Path::Own) walked(tree_multT_[ix], out + 2);
+  if (mult_path_ != Path::Own && multT_path_ != Path::Own) return;
   check_hip(hipSetDevice(device_), "hipSetDevice");
   const size_t n = std::max(N_, M_) * sizeof(double);
   ensure(&hin_, &hin_cap_, n);
@@ -907,7 +910,8 @@ void DeviceMultiEval::count_work(Precision p, uint64_t out[4]) {
     unsigned long long h[4];
     check_hip(hipMemcpyAsync(h, dcnt, sizeof(h), hipMemcpyDeviceToHost, stream_), "read counters");
     check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-    for (int i = 0; i < 4; ++i) out[i] = h[i];
+    for (int i = 0; i < 4; ++i)
+      if ((i < 2 ? mult_path_ : multT_path_) == Path::Own) out[i] = h[i];
   } catch (...) {
     count_ = nullptr;
     timing_on_ = timing;
@@ -917,16 +921,23 @@ void DeviceMultiEval::count_work(Precision p, uint64_t out[4]) {
   }
   timing_on_ = timing;
   check_hip(hipFree(dcnt), "hipFree(counters)");
-  if (mult_path_ != Path::Own) out[0] = out[1] = walked;
-  if (multT_path_ != Path::Own) out[2] = out[3] = walked;
   if (D_ > static_cast<size_t>(kMaxTemplD)) {
     // the generic kernels evaluate every pair of the padded arrays in every dimension
-    const uint64_t jend = static_cast<uint64_t>(ceil_div(N_, kTG)) * kTG;
-    out[1] = static_cast<uint64_t>(Mpad_) * jend;
-    out[0] = out[1] * D_;
-    out[3] = out[1];
-    out[2] = out[0];
+    const uint64_t pairs = static_cast<uint64_t>(Mpad_) * ceil_div(N_, kTG) * kTG;
+    for (int i = 0; i < 4; ++i)
+      if ((i < 2 ? mult_path_ : multT_path_) == Path::Own) out[i] = i % 2 ? pairs : pairs * D_;
   }
+}
+
+const char* DeviceMultiEval::kernel_name(bool multT) const {
+  if (N_ == 0) throw input_error("grid not set (call prepare)");
+  if ((multT ? multT_path_ : mult_path_) == Path::Tree)
+    return multT ? "tree_multT_kernel" : "tree_mult_kernel";
+  if (algorithm_ == Algorithm::Subspace)
+    return multT ? "subspace_multT_kernel" : "subspace_mult_kernel";
+  if (D_ > static_cast<size_t>(kMaxTemplD))
+    return multT ? "multT_kernel_generic" : "mult_kernel_generic";
+  return multT ? "multT_kernel" : "mult_kernel";
 }
 
 DeviceMultiEval::EventPair* DeviceMultiEval::next_timer(std::vector<EventPair>& pool,

@@ -344,6 +344,10 @@ int64_t tree_walks(const TreeGrid& g, bool multT) {
 
 void DeviceMultiEval::upload_tree(const TreeProgram& p, TreePlan& plan, int entry_bytes) {
   plan.ngroups = static_cast<int>(p.groups.size()) - 1;
+  plan.factors = static_cast<int64_t>(p.recs.size()) - 1;
+  plan.lookups = 0;
+  for (const TreeRec& r : p.recs) plan.lookups += (r.ctl & (kTreeTable | kTreePart)) != 0;
+  for (const TreeChunk& c : p.chunks) plan.lookups += c.root;
   plan.lds = (p.max_entries * entry_bytes + 15) / 16 * 16;
   ensure(&plan.recs, &plan.recs_cap, p.recs.size() * sizeof(TreeRec));
   check_hip(hipMemcpy(plan.recs, p.recs.data(), p.recs.size() * sizeof(TreeRec),
@@ -529,7 +533,6 @@ bool DeviceMultiEval::set_tree(const TreeGrid& g, const uint32_t* level, const u
   check_hip(hipMemcpy(tree_ti_, ti.data(), ti.size() * sizeof(int32_t), hipMemcpyHostToDevice),
             "upload tables");
   tree_total_ = g.total;
-  tree_nodes_ = static_cast<int64_t>(g.node.size());
   tree_depth_ = g.depth;
   if (serves(Precision::FP64)) set_tree_plans<double>(g, mult, multT);
   if (serves(Precision::FP32)) set_tree_plans<float>(g, mult, multT);

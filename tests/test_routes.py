@@ -100,3 +100,43 @@ for algorithm in (0, 1):
     most = grids(mult_grid_chunks=1000000, multT_data_segs=1000000, algorithm=algorithm)
     assert most["allocated"] <= 2 * (2048 << 20) + (64 << 20), most
 """)
+
+
+def test_kernels_and_work_of_walks(on_host):
+    """The kernels' names, and a walk's executed work: every data row, the padding to whole blocks
+    included, looks each subspace up once, one of 2^13 cells in its parts (of 5,119 entries in FP64;
+    of 1,280 in multTranspose); factors are at least the subspaces' but the root's."""
+    on_host(GRIDS + """
+def names(op):
+    out = []
+    for call, n in ((op.mult, op.N), (op.mult_transpose, op.M)):
+        launches()
+        call(np.zeros(n))
+        out.append(" ".join(name for name, _, _, _ in launches()))
+    return out
+
+fine = np.ones((1 << 13, 3), np.uint32), np.ones((1 << 13, 3), np.uint32)
+fine[0][:, 0], fine[1][:, 0] = 14, 2 * np.arange(1 << 13) + 1
+lv, ix = regular(3, 5)  # 35 subspaces
+for grid, mult, multT in (((lv, ix), 35, 35),
+                          ((np.concatenate([lv, fine[0]]), np.concatenate([ix, fine[1]])), 37, 42)):
+    op = capi.MultiEval(0, uniform(5000, 3)).prepare(*grid)
+    assert op.kernels() == ("tree_mult_kernel", "tree_multT_kernel")
+    w, rows = op.count_work(0), 5120  # one point per lane
+    assert w["mult_pairs"] == rows * mult and w["multT_pairs"] == rows * multT, w
+    assert rows * 34 <= w["mult_hat_steps"] <= 3 * rows * mult, w
+
+repeated = np.concatenate([lv, lv[:1]]), np.concatenate([ix, ix[:1]])
+for algorithm in (0, 1):
+    for grid in ((lv, ix), repeated):
+        op = capi.MultiEval(0, uniform(5000, 3), algorithm=algorithm).prepare(*grid)
+        assert all(k in n for k, n in zip(op.kernels(), names(op))), (op.kernels(), names(op))
+lv, ix = regular(24, 2)
+op = capi.MultiEval(0, uniform(50, 24)).prepare(np.concatenate([lv, lv[:1]]), np.concatenate([ix, ix[:1]]))
+assert op.kernels() == ("mult_kernel_generic", "multT_kernel_generic") and "generic" in names(op)[1]
+try:
+    capi.MultiEval(0, uniform(50, 3)).kernels()
+    raise AssertionError("named kernels without a grid")
+except capi.SGppHIPError:
+    pass
+""")
