@@ -60,6 +60,8 @@ constexpr int kTreePassShift = 24;          // 4 bits: the dimensions before the
 //   d=2  level 8     0.49  0.42  0.98     d=11 20,000 points  1.59  1.31  1.47
 //   d=5  level 7     0.98  0.84  1.30     d=20 level 4        3.26  1.80  1.64
 //   d=9  20,000 points 1.42 1.22 1.56     d=30 level 3        3.68  2.17  0.92
+// (Taken out of a product of all below 2^-126, FP32 values lose digits: basis values
+// below 2^-96; a coordinate below 2^-127 counts as 0.)
 constexpr int kTreePassDims = 10;
 
 struct alignas(16) TreeRec {

@@ -44,8 +44,8 @@ __global__ void tree_points_kernel(const T* __restrict__ X, int64_t ldx,
                                    const int32_t* __restrict__ dperm, int64_t M, int D, int K,
                                    int64_t rows, T* __restrict__ XT,
                                    int32_t* __restrict__ sperm) {
-  // (below this a Linear level-1 factor's reciprocal could overflow)
-  constexpr double kTiny = sizeof(T) == 4 ? 0x1.0p-100 : 0x1.0p-1000;
+  // (below this the reciprocal of a halved level-1 factor could overflow)
+  constexpr double kTiny = sizeof(T) == 4 ? 0x1.0p-127 : 0x1.0p-1023;
   const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (r >= rows) return;
   constexpr int kGroup = 1 << kTreeJoin, kGroups = 64 / kGroup;
@@ -65,7 +65,7 @@ __global__ void tree_points_kernel(const T* __restrict__ X, int64_t ldx,
     if (pass) {
       XT[(D + d) * rows + r] = static_cast<T>(all.value());
     } else {
-      if (2.0 * half < kTiny) half = 0.0;
+      if (half < kTiny) half = 0.0;
       XT[(D + d) * rows + r] = static_cast<T>(half == 0.0 ? 0.0 : 1.0 / half);
     }
     all.times(half);

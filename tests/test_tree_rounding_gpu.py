@@ -5,8 +5,6 @@ takes a Linear level-1 factor out of a product of all, one and three per refined
 import numpy as np
 import pytest
 
-pytestmark = pytest.mark.gpu
-
 
 def basis_value(basis, X, lv, ix):
     p = np.ones(len(X), np.longdouble)
@@ -24,6 +22,7 @@ def basis_value(basis, X, lv, ix):
     return p
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("basis", [0, 1])
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("d,level", [(1, 8), (2, 8), (3, 6), (4, 5), (5, 5), (8, 4), (10, 3), (11, 4), (20, 3), (30, 3)])
@@ -52,3 +51,24 @@ def test_roundings(gpu, basis, prec, d, level):
         got = op.mult_transpose(e).astype(np.longdouble)
         for j in rng.choice(len(lv), 40):
             check(got[j], basis_value(basis, X[m:m + 1], lv[j], ix[j])[0], (lv[j] > 1).sum())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("d", [3, 11, 24])
+def test_small_coordinates(gpu, prec, d):
+    """A coordinate far below the finest cell: the values are small, not 0."""
+    capi = gpu
+    lv, ix = np.ones((2, d), np.uint32), np.ones((2, d), np.uint32)
+    lv[1, 0] = 12
+    x0 = 2.0 ** -np.array([30, 60, 90, 100, 101, 110, 114])
+    X = np.full((len(x0), d), 0.375)
+    X[:, 0] = x0
+    op = capi.MultiEval(0, X, precision=prec).prepare(lv, ix)
+    u, n = 2.0 ** (-24 if prec else -53), max(d - 1, 4)
+    for j, l in ((0, 1), (1, 12)):
+        exact = x0 * 2.0 ** l * 0.75 ** (d - 1)
+        assert np.all(exact > 2.0 ** -126)
+        e = np.zeros(2)
+        e[j] = 1.0
+        assert np.all(abs(op.mult(e) - exact) <= 2 * n * u * exact)
