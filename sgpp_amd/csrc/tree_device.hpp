@@ -41,14 +41,13 @@ constexpr int kTreeBlock = 256;
 constexpr int kTreeJoin = 1;
 
 // ctl of a record
-constexpr uint32_t kTreeShiftMask = 31u;    // 33 - level
+// bits 0 to 4: 33 - level
 constexpr int kTreeDimShift = 8;            // 6 bits: the dimension
 constexpr uint32_t kTreeRun = 1u << 16;     // first of its (parent, dimension): fetch its values
 constexpr uint32_t kTreeTable = 1u << 17;   // the subspace has grid points (absent parents are walked without)
 constexpr uint32_t kTreePush = 1u << 18;    // children follow
 constexpr uint32_t kTreeLast = 1u << 19;    // last of its parent's children
 constexpr uint32_t kTreeFlush = 1u << 20;   // add the FP32 sums to the FP64 ones
-
 constexpr uint32_t kTreePart = 1u << 21;    // (without kTreeTable) part of a table: see TreeChunk
 constexpr int kTreePassShift = 24;          // 4 bits: the dimensions before the run's to pass first
 
@@ -74,14 +73,13 @@ static_assert(sizeof(TreeRec) == 16, "one record is 16 bytes");
 
 // A run of consecutive subspaces whose tables fit the LDS image: records
 // [rec0, rec0 + nrec), table entries [off0, off0 + n). root: the chunk begins
-// with the subspace of level 1 in every dimension (one entry, the first).
-// part: one subspace whose table exceeds the image; the chunk holds its
-// positions [part0, part0 + n).
+// with the subspace of level 1 in every dimension (one entry, the first). Of a
+// subspace whose table exceeds the image a chunk holds positions [part0, part0 + n).
 struct alignas(16) TreeChunk {
   int rec0, nrec;
   int n, part0;
   long long off0;
-  int root, part;
+  int root, pad;
 };
 static_assert(sizeof(TreeChunk) == 32, "one chunk is 32 bytes");
 
