@@ -451,7 +451,7 @@ void DeviceMultiEval::set_grid(const uint32_t* level, const uint32_t* index, siz
 // What the kernels of the instance's algorithm take, in us, to be held against
 // tree_times(). Fitted to 842 pairs of both (each basis, precision and algorithm; 1 to 60
 // dimensions, 41 to 100,000 grid points, 300 to 8e6 data points). The kernels
-// chosen by the fits take 1.2 % more than the faster ones of each pair.
+// chosen by the fits take 1.4 % more than the faster ones of each pair.
 //
 // Culled: a cost per data point, the grid points that a data group's box meets (two
 // per evaluated dimension and 2.5 more), estimated on a few groups and grid points, and

@@ -387,20 +387,22 @@ bool DeviceMultiEval::tree_wide(const TreeGrid& g) const {
 // The walks' times, fitted to the same pairs as own_times(): a launch or three; per
 // data point and node (parts of a table are walked each, with adds that meet in
 // multTranspose; walks of more than tree_few_dims() refined dimensions take one
-// point per lane, those of more than kRegDims dimensions read them from memory); what a block of mult
-// copies of the tables, and the chain of one table's parts; multTranspose's partial
-// sums and the rows that a final sum adds.
+// point per lane, those of more than kRegDims dimensions read them from memory) and per
+// data point; what a block of mult copies of the tables, and the chain of one table's
+// parts; multTranspose's partial sums and the rows that a final sum adds.
 DeviceMultiEval::PathTimes DeviceMultiEval::tree_times(const TreeGrid& g) const {
   constexpr size_t kRegDims = 20;  // (of tree_launch)
-  // 1e-6 us per data point and node, mult and multTranspose: up to 10 dimensions,
-  // more, deep, more than kRegDims
-  constexpr double kNode[2][4][2] = {{{0.58, 1.11}, {0.77, 1.42}, {0.98, 1.54}, {1.3, 2.6}},
-                                     {{0.36, 0.67}, {0.42, 0.81}, {0.87, 1.35}, {0.9, 1.6}}};
+  // 1e-6 us per data point and node, mult and multTranspose: up to 10 dimensions
+  // (Linear, ModLinear), more, deep, more than kRegDims; per data point (multTranspose)
+  constexpr double kNode[2][5][2] = {
+      {{0.55, 1.11}, {0.51, 0.83}, {0.73, 1.28}, {0.8, 1.45}, {1.25, 2.0}},
+      {{0.33, 0.6}, {0.345, 0.52}, {0.4, 0.7}, {0.76, 1.24}, {0.9, 1.4}}};
+  constexpr double kPoint[5] = {30.0, 30.0, 100.0, 35.0, 50.0};
   const bool fp32 = serves(Precision::FP32), mod = basis_ == Basis::ModLinear;
   const bool wide = fp32 ? tree_wide<float>(g) : tree_wide<double>(g);
   const TreeLaunch l = fp32 ? tree_variant_of<float>(mod, D_, g.depth, wide)
                             : tree_variant_of<double>(mod, D_, g.depth, wide);
-  const int c = D_ > kRegDims ? 3 : (g.depth > tree_few_dims(D_) ? 2 : (D_ > 10 ? 1 : 0));
+  const int c = D_ > kRegDims ? 4 : (g.depth > tree_few_dims(D_) ? 3 : (D_ > 10 ? 2 : mod));
   const double M = static_cast<double>(M_), nodes = static_cast<double>(g.node.size()),
                total = static_cast<double>(g.total),
                walks = static_cast<double>(tree_walks(g, false)),
@@ -409,8 +411,8 @@ DeviceMultiEval::PathTimes DeviceMultiEval::tree_times(const TreeGrid& g) const 
   const double rows = std::min(M / (64 * l.k), 24576.0 / std::max(1.0, total / kMultTEntries));
   return {20.0 + 1e-6 * (kNode[fp32][c][0] * walks + 8.0) * M + 1.2e-6 * total * blocks +
               50e-6 * total + 0.25 * (walks - nodes),
-          25.0 + 1e-6 * (kNode[fp32][c][1] * (2.0 * walksT - nodes) + 15.0) * M + 25e-6 * total +
-              0.015 * rows};
+          26.0 + 1e-6 * (kNode[fp32][c][1] * (2.0 * walksT - nodes) + kPoint[c]) * M +
+              25e-6 * total + 0.015 * rows};
 }
 
 template <typename T>
