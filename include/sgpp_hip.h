@@ -115,8 +115,8 @@ typedef struct sgpp_hip_params {
  *   operation/hash/OperationMultipleEvalSubspace/combined/
  *   OperationMultipleEvalSubspaceCombined.hpp:92-204). FP64 only
  *   (precision SGPP_HIP_PREC_FP64, keep_fp64 0), dimension <= 20, Linear and
- *   ModLinear; multiTranspose sums with FP64 atomics, so its last bits vary
- *   between runs. Grids whose index tables would exceed
+ *   ModLinear; where its own kernels run, multTranspose sums with FP64 atomics
+ *   and its last bits vary between runs. Grids whose index tables would exceed
  *   max(2^26, 64 N) entries are refused. */
 enum { SGPP_HIP_ALGO_STREAMING = 0, SGPP_HIP_ALGO_SUBSPACE = 1 };
 

@@ -301,9 +301,9 @@ struct TreeGather {
 };
 
 // mult: bound by vector instructions, most of which issue every four cycles in
-// either precision: seven (Linear) or nine per node and data point and four per run
-// (one scalar instruction issues in four cycles, so several points per lane share
-// a node's). The weights of a chunk's subspaces are gathered from LDS, where up to
+// either precision: seven (Linear) or nine per node and data point, four per run and
+// five per dimension passed (one scalar instruction issues in four cycles, so several
+// points per lane share a node's). The weights of a chunk's subspaces are gathered from LDS, where up to
 // 64 cells meet no bank conflict. Kernel times against the culled kernels: Linear
 // d=8 level 6, 5e5 points, FP32 1,179 to 260 us, FP64 1,678 to 403; d=20 adaptive,
 // 5e5 points, FP32 6,523 to 3,023; ModLinear d=10 adaptive, 1e6 points, FP32 2,051
